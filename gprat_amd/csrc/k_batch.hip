@@ -33,16 +33,15 @@ using blk::v4d;
 
 typedef double d2 __attribute__((ext_vector_type(2)));
 
-struct Stage
+struct alignas(16) Stage
 {
     double a[NB * XS];
     double b[NB * XS];
 };
-struct Factor
+struct alignas(16) Factor
 {
-    double D[NB][NB + 1];
-    double W[NB][NB + 1];
-    double R[NB];
+    double D[NB][XS];
+    double W[NB][XS];
     double T[NB];  // the diagonal step's L_jb,0:jb z_0:jb (alpha's forward solve)
 };
 // FP32 copies of two 64x64 blocks for the mixed-precision products; row
@@ -657,7 +656,7 @@ __device__ __forceinline__ void diag_block(const BatchGP &g, int gi, int jb, Sha
         sh.fa.D[r][c] = (c <= r) ? kij[q] : 0.0;
     }
     __syncthreads();
-    factor_block64(sh.fa.D, sh.fa.W, sh.fa.R, info + gi, jb * NB);
+    factor_block64(sh.fa.D, sh.fa.W, info + gi, jb * NB);
     double *Cjj = g.L + static_cast<long>(jb) * NB * np + jb * NB;
     double *Wjj = g.W + static_cast<long>(jb) * NB * NB;
     for (int e = threadIdx.x; e < NB * NB; e += THREADS)
@@ -1269,7 +1268,7 @@ __device__ __forceinline__ void diag_block128(const BatchGP &g, int gi, int jb, 
         sh.fa.D[r][c] = (c <= r) ? C[static_cast<long>(r) * np + c] : 0.0;
     }
     __syncthreads();
-    factor_block64(sh.fa.D, sh.fa.W, sh.fa.R, info + gi, static_cast<int>(j0));
+    factor_block64(sh.fa.D, sh.fa.W, info + gi, static_cast<int>(j0));
     for (int e = tid; e < NB * NB; e += THREADS)
     {
         const int r = e / NB, c = e % NB;
@@ -1311,7 +1310,7 @@ __device__ __forceinline__ void diag_block128(const BatchGP &g, int gi, int jb, 
                       q++;
                   });
     __syncthreads();
-    factor_block64(sh.fa.D, sh.fa.W, sh.fa.R, info + gi, static_cast<int>(j0 + NB));
+    factor_block64(sh.fa.D, sh.fa.W, info + gi, static_cast<int>(j0 + NB));
     for (int e = tid; e < NB * NB; e += THREADS)
     {
         const int r = e / NB, c = e % NB;

@@ -17,7 +17,7 @@ constexpr int THREADS = 256;
 
 // Lower triangle of the NB x NB block at (r0, r0) into LDS (strict upper
 // zeroed); every load of a thread is issued before the first LDS store.
-__device__ __forceinline__ void load_lower_block(const double *__restrict__ A, long lda, long r0, double (*D)[NB + 1])
+__device__ __forceinline__ void load_lower_block(const double *__restrict__ A, long lda, long r0, double (*D)[blk::XS])
 {
     double v[NB * NB / THREADS];
 #pragma unroll
@@ -60,10 +60,10 @@ __device__ __forceinline__ double *blockW(const PanelArgs &a, int i, int j) { re
 // FACTOR / UFACTOR: block (k, k) (minus L_kq L_kq^T when q >= 0) factored
 // and inverted in LDS; L to A (lower triangle), the inverse to Winv_k
 // (row-major, zero upper).
-__device__ __noinline__ void task_factor(const PanelArgs &a, int k, int q, double *buf0, double *buf1, double *R)
+__device__ __noinline__ void task_factor(const PanelArgs &a, int k, int q, double *buf0, double *buf1)
 {
-    double(*D)[NB + 1] = reinterpret_cast<double(*)[NB + 1]>(buf0);
-    double(*Wl)[NB + 1] = reinterpret_cast<double(*)[NB + 1]>(buf1);
+    double(*D)[blk::XS] = reinterpret_cast<double(*)[blk::XS]>(buf0);
+    double(*Wl)[blk::XS] = reinterpret_cast<double(*)[blk::XS]>(buf1);
     double *blk = blockA(a, k, k);
     load_lower_block(blk, a.h.lda, 0, D);
     if (q >= 0)
@@ -80,7 +80,7 @@ __device__ __noinline__ void task_factor(const PanelArgs &a, int k, int q, doubl
                       });
     }
     __syncthreads();  // D final; every read of buf1 done before W lands there
-    factor_block64(D, Wl, R, a.h.info, static_cast<int>(a.h.p0) + NB * k);
+    factor_block64(D, Wl, a.h.info, static_cast<int>(a.h.p0) + NB * k);
     double *w = blockWinv(a, k);
     for (int e = threadIdx.x; e < NB * NB; e += THREADS)
     {
@@ -233,9 +233,8 @@ __device__ __noinline__ void task_heads(const PanelArgs &a, int i, int j, double
 
 __global__ __launch_bounds__(THREADS) void k_panel_tasks(PanelArgs a)
 {
-    __shared__ double buf0[NB * blk::XS];
-    __shared__ double buf1[NB * blk::XS];
-    __shared__ double R[NB];
+    __shared__ alignas(16) double buf0[NB * blk::XS];
+    __shared__ alignas(16) double buf1[NB * blk::XS];
     const int first = a.wg_off[blockIdx.x], last = a.wg_off[blockIdx.x + 1];
     for (int t = first; t < last; t++)
     {
@@ -243,7 +242,7 @@ __global__ __launch_bounds__(THREADS) void k_panel_tasks(PanelArgs a)
         const int type = d.x & 0xff;
         __syncthreads();  // the previous task's LDS reads are done
         if (type == PT_FACTOR || type == PT_UFACTOR)
-            task_factor(a, d.y, type == PT_UFACTOR ? d.z : -1, buf0, buf1, R);
+            task_factor(a, d.y, type == PT_UFACTOR ? d.z : -1, buf0, buf1);
         else if (type == PT_SOLVE)
             task_solve(a, d.y, d.z, buf0, buf1);
         else if (type == PT_UPDATE)
