@@ -13,6 +13,9 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 
 constexpr int NB = 64;
 constexpr int THREADS = 256;
+// (The thread's index is a parameter so that a kernel which runs many block
+// operations in one loop can hide it from the compiler, which otherwise keeps
+// every operation's addresses across the loop, in scratch.)
 constexpr int XS = NB + 2;  // LDS row stride of staged blocks (bank-spread MFMA reads)
 
 typedef double d2 __attribute__((ext_vector_type(2)));
@@ -20,19 +23,19 @@ typedef double d2 __attribute__((ext_vector_type(2)));
 // Copy a 64x64 row-major block (leading dimension ld) into LDS stride XS:
 // all eight 16-byte loads of a thread are issued before the first LDS
 // store, so the block costs one memory latency, not eight.
-__device__ __forceinline__ void stage_block(double *dst, const double *__restrict__ src, long ld)
+__device__ __forceinline__ void stage_block(double *dst, const double *__restrict__ src, long ld, int tid = threadIdx.x)
 {
     d2 v[8];
 #pragma unroll
     for (int s = 0; s < 8; s++)
     {
-        const int e = threadIdx.x + THREADS * s;
+        const int e = tid + THREADS * s;
         v[s] = *reinterpret_cast<const d2 *>(src + static_cast<long>(e >> 5) * ld + (e & 31) * 2);
     }
 #pragma unroll
     for (int s = 0; s < 8; s++)
     {
-        const int e = threadIdx.x + THREADS * s;
+        const int e = tid + THREADS * s;
         *reinterpret_cast<d2 *>(dst + (e >> 5) * XS + (e & 31) * 2) = v[s];
     }
 }
@@ -62,22 +65,22 @@ __device__ __forceinline__ void stage_block_t(double *dst, const double *__restr
 // block can be in flight while the current one is multiplied: load_block
 // issues this thread's eight 16-byte loads, store_block / store_block_t
 // write them to LDS (stride XS; transposed: dst[c][r] = src[r][c]).
-__device__ __forceinline__ void load_block(const double *__restrict__ src, long ld, d2 (&v)[8])
+__device__ __forceinline__ void load_block(const double *__restrict__ src, long ld, d2 (&v)[8], int tid = threadIdx.x)
 {
 #pragma unroll
     for (int s = 0; s < 8; s++)
     {
-        const int e = threadIdx.x + THREADS * s;
+        const int e = tid + THREADS * s;
         v[s] = *reinterpret_cast<const d2 *>(src + static_cast<long>(e >> 5) * ld + (e & 31) * 2);
     }
 }
 
-__device__ __forceinline__ void store_block(double *dst, const d2 (&v)[8])
+__device__ __forceinline__ void store_block(double *dst, const d2 (&v)[8], int tid = threadIdx.x)
 {
 #pragma unroll
     for (int s = 0; s < 8; s++)
     {
-        const int e = threadIdx.x + THREADS * s;
+        const int e = tid + THREADS * s;
         *reinterpret_cast<d2 *>(dst + (e >> 5) * XS + (e & 31) * 2) = v[s];
     }
 }
@@ -106,9 +109,9 @@ __device__ __forceinline__ void zero(v4d (&acc)[2][2])
 // acc (this wavefront's 32x32 quarter of a 64x64 block) += sum_k A[r][k] B[c][k]
 // with A and B staged in LDS (stride XS). Wavefront w owns rows
 // 32*(w>>1).., columns 32*(w&1)..
-__device__ __forceinline__ void mfma_nt_acc(const double *A, const double *B, v4d (&acc)[2][2])
+__device__ __forceinline__ void mfma_nt_acc(const double *A, const double *B, v4d (&acc)[2][2], int tid = threadIdx.x)
 {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid & 63, w = tid >> 6;
     const int lm = lane & 15, lk = lane >> 4;
     const int r0 = (w >> 1) * 32, c0 = (w & 1) * 32;
 #pragma unroll 4
@@ -215,9 +218,9 @@ __device__ __forceinline__ void mfma_nt(const double *A, const double *B, v4d (&
 // 64x64 block. f64 16x16x4 accumulator layout (measured on gfx950): lane
 // holds column lane%16, rows lane/16 + 4e.
 template <class F>
-__device__ __forceinline__ void for_each(const v4d (&acc)[2][2], F f)
+__device__ __forceinline__ void for_each(const v4d (&acc)[2][2], F f, int tid = threadIdx.x)
 {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid & 63, w = tid >> 6;
     const int lm = lane & 15, lk = lane >> 4;
     const int r0 = (w >> 1) * 32, c0 = (w & 1) * 32;
 #pragma unroll
@@ -232,9 +235,9 @@ __device__ __forceinline__ void for_each(const v4d (&acc)[2][2], F f)
 // The 16 entries of a 64x64 global block (leading dimension ld) at this
 // lane's accumulator positions, in for_each order; all loads are issued
 // before any is used.
-__device__ __forceinline__ void load_at_acc(const double *__restrict__ C, long ld, double (&v)[16])
+__device__ __forceinline__ void load_at_acc(const double *__restrict__ C, long ld, double (&v)[16], int tid = threadIdx.x)
 {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = tid & 63, w = tid >> 6;
     const int lm = lane & 15, lk = lane >> 4;
     const int r0 = (w >> 1) * 32, c0 = (w & 1) * 32;
 #pragma unroll

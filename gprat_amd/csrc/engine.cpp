@@ -216,6 +216,7 @@ Context::Context(int dev, int ns) : device(dev), n_streams(ns), pool(dev)
         GP_HIP(hipStreamCreateWithFlags(&panel, hipStreamNonBlocking));
     info = DevBuf<int>(*this, 1);
     scalars = DevBuf<double>(*this, 64);
+    GP_HIP(hipHostMalloc(reinterpret_cast<void **>(&host_info), sizeof(int), hipHostMallocDefault));
     k::noalloc_scratch_init(device);
 }
 
@@ -234,6 +235,8 @@ Context::~Context()
     batch_graphs.clear();
     info.reset();
     scalars.reset();
+    if (host_info)
+        hipHostFree(host_info);
     if (trail && trail != main)
         hipStreamDestroy(trail);
     if (panel && panel != main)
@@ -450,14 +453,67 @@ const Context::PanelPlanDev &Context::cached_plan(long key, const std::function<
 // step k-1's update has reached it) and factors that block, while the
 // `trail` stream solves panel k's rows and applies panel k to everything
 // below block k+1.
+// Sizes the dataflow launch factors faster than the panel schedule.
+// Measured on MI355X (whole FP64 fit, panels / dataflow, ms): n = 1024
+// 0.82 / 0.42, 4096 3.58 / 2.01, 8192 9.26 / 6.45, 10240 13.6 / 11.1, 12288
+// 19.7 / 18.3, 14336 27.2 / 28.3, 16384 36.9 / 42.0: beyond, its 64x64 tiles
+// reuse an operand too little. A mixed-precision fit whose whole factor is
+// FP64 on this path is faster than with FP32 trailing updates up to n = 10240
+// (2048 2.09 / 1.07, 8192 9.8 / 7.1, 10240 13.2 / 11.9, 12288 16.9 / 19.3).
+// GPRAT_FLOW_LIMIT overrides, and the panel
+// schedule's own overrides ask for that schedule.
+constexpr int FLOW_LIMIT = 12288, FLOW_LIMIT_MIXED = 10240;
+bool one_launch(int n_pad, bool mixed)
+{
+    if (std::getenv("GPRAT_CHOLESKY_BLOCK") || std::getenv("GPRAT_LOOKAHEAD"))
+        return false;
+    if (const char *e = std::getenv("GPRAT_FLOW_LIMIT"))
+        return n_pad <= std::atoi(e);
+    return n_pad <= (mixed ? FLOW_LIMIT_MIXED : FLOW_LIMIT);
+}
+
+void check_pivots(Context &c)
+{
+    const int info = *c.host_info;
+    if (info == k::FLOW_STALLED)
+        throw Error(GPRAT_ERR_INTERNAL, "factorisation: a tile was never finished");
+    if (info != INT_MAX)
+        throw Error(GPRAT_ERR_NOT_SPD,
+                    "covariance matrix is not positive definite (first non-positive pivot at column "
+                        + std::to_string(info) + ")");
+}
+
+// The factorisation as one launch, then the panels' whole inverses if they
+// are kept.
+static void flow(Context &c, double *A, long lda, int n_pad, double *Winv, double *Wpanel, double *X, int extra, bool unit = false)
+{
+    Timed t(c, c.main, "cholesky");
+    const int nb = n_pad / 64, ne = extra / 64;
+    DevBuf<int> counters(c, static_cast<std::size_t>(k::flow_counters(nb, ne)));
+    k::flow_cholesky(c.main, k::FlowCall{ A, lda, X, nb, ne, unit, Winv, c.info.get(), counters.get() }, c.cus);
+    if (Wpanel)
+    {
+        const int width = outer_block(n_pad);
+        DevBuf<double> tmp(c, static_cast<std::size_t>(std::max(1L, k::panel_inverses_scratch(n_pad, width))));
+        k::panel_inverses(c.main, A, lda, Winv, n_pad, width, Wpanel, tmp.get());
+    }
+    GP_HIP(hipMemcpyAsync(c.host_info, c.info.get(), sizeof(int), hipMemcpyDeviceToHost, c.main));
+}
+
 void cholesky_fp64(Context &c, double *A, long lda, int n_pad, double *Winv) { cholesky(c, A, lda, n_pad, Winv, false); }
 
 int panel_width(int n_pad) { return outer_block(n_pad); }
 
-void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel, int extra)
+void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel, int extra, double *X)
 {
     require(n_pad % 128 == 0 && lda >= n_pad && lda % 2 == 0, "cholesky: bad layout");
     require(extra >= 0 && extra % 64 == 0, "cholesky: extra rows must come in 64s");
+    if (one_launch(n_pad, mixed))
+    {
+        flow(c, A, lda, n_pad, Winv, Wpanel, X ? X : A + static_cast<long>(n_pad) * lda, extra);
+        return;
+    }
+    require(X == nullptr, "cholesky: the panel schedule takes its rows below the matrix");
     // rows of L and the rows below it that ride along (right-hand sides)
     const long rows = static_cast<long>(n_pad) + extra;
     const bool ahead = use_lookahead() && c.panel != c.main;
@@ -621,15 +677,24 @@ void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mix
         wait(c.main, record(T), T);
         wait(c.main, record(P), P);
     }
+    GP_HIP(hipMemcpyAsync(c.host_info, c.info.get(), sizeof(int), hipMemcpyDeviceToHost, c.main));
     c.sync();
     for (auto e : used)
         c.recycle(e);
-    int info = INT_MAX;
-    GP_HIP(hipMemcpy(&info, c.info.get(), sizeof(int), hipMemcpyDefault));
-    if (info != INT_MAX)
-        throw Error(GPRAT_ERR_NOT_SPD,
-                    "covariance matrix is not positive definite (first non-positive pivot at column "
-                        + std::to_string(info) + ")");
+    check_pivots(c);
+}
+
+// out = L^-T z with the panels' kept inverses; z is overwritten.
+static void solve_upper(Context &c, const double *L, long lda, int n_pad, double *z, double *out, const double *Wpanel, int wblock)
+{
+    const int nblk = static_cast<int>(ceil_div(n_pad, wblock));
+    for (int J = nblk - 1; J >= 0; J--)
+    {
+        const int j0 = J * wblock, nb = std::min(wblock, n_pad - j0);
+        k::rowdot(c.main, Wpanel + static_cast<long>(J) * wblock * wblock, wblock, nb, nb, z + j0, out + j0, false);
+        if (j0 > 0)
+            k::coldot(c.main, L + static_cast<long>(j0) * lda, lda, nb, j0, out + j0, z, true);
+    }
 }
 
 // alpha = K^-1 y by the blocked forward and backward solves. With the
@@ -656,14 +721,8 @@ void solve_spd(Context &c, const double *L, long lda, const double *Winv, int n_
             if (j1 < n_pad)
                 k::rowdot(s, L + static_cast<long>(j1) * lda + j0, lda, nb, n_pad - j1, out + j0, work + j1, true);
         }
-        // out holds z = L^-1 y, updated in place; x = L^-T z goes to work
-        for (int J = nblk - 1; J >= 0; J--)
-        {
-            const int j0 = J * wblock, nb = std::min(wblock, n_pad - j0);
-            k::rowdot(s, WJ(J), wblock, nb, nb, out + j0, work + j0, false);
-            if (j0 > 0)
-                k::coldot(s, L + static_cast<long>(j0) * lda, lda, nb, j0, work + j0, out, true);
-        }
+        // out holds z = L^-1 y
+        solve_upper(c, L, lda, n_pad, out, work, Wpanel, wblock);
     }
     else
     {
@@ -1083,13 +1142,19 @@ static void upload(Context &c, double *dst, const double *src, std::size_t count
         GP_HIP(hipMemcpyAsync(dst, src, count * sizeof(double), hipMemcpyDefault, c.main));
 }
 
-void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int r, const double theta[3], int precision)
+static void check_training(const double *x, std::size_t x_len, int n, int r, const double *theta, int precision)
 {
     require(n >= 1, "need at least one training point");
     require(r >= 1, "n_reg must be >= 1");
     require(x != nullptr && x_len >= static_cast<std::size_t>(n) + r - 1, "training input must hold n + n_reg - 1 values");
     require(theta != nullptr, "theta is null");
     require(precision == GPRAT_PRECISION_FP64 || precision == GPRAT_PRECISION_MIXED, "unknown precision mode");
+}
+
+void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int r, const double theta[3], int precision, double *rhs,
+            bool keep_inverses)
+{
+    check_training(x, x_len, n, r, theta, precision);
     c.make_current();
     m.ctx = &c;
     m.n = n;
@@ -1103,13 +1168,15 @@ void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int
     m.L = DevBuf<double>(c, static_cast<std::size_t>(m.n_pad) * m.lda);
     m.Winv = DevBuf<double>(c, static_cast<std::size_t>(m.n_pad) * 64);
     m.wblock = panel_width(m.n_pad);
-    m.Wpanel = DevBuf<double>(c, static_cast<std::size_t>(ceil_div(m.n_pad, m.wblock)) * m.wblock * m.wblock);
+    if (keep_inverses)
+        m.Wpanel = DevBuf<double>(c, static_cast<std::size_t>(ceil_div(m.n_pad, m.wblock)) * m.wblock * m.wblock);
     upload(c, m.x.get(), x, xl);
     {
         Timed t(c, c.main, "assemble");
         k::assemble_lower(c.main, m.x.get(), r, m.sek, m.L.get(), m.lda, n, m.n_pad);
     }
-    cholesky(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), precision == GPRAT_PRECISION_MIXED, m.Wpanel.get());
+    cholesky(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), precision == GPRAT_PRECISION_MIXED, m.Wpanel.get(),
+             rhs ? 64 : 0, rhs);
     if (precision == GPRAT_PRECISION_MIXED)
     {
         // the covariance's strictly lower part, for the FP64 residual of the
@@ -1172,22 +1239,6 @@ void refine_alpha(Model &m, double *work)
     }
 }
 
-void attach_targets(Model &m, const double *y, std::size_t y_len)
-{
-    Context &c = *m.ctx;
-    require(y != nullptr && y_len >= static_cast<std::size_t>(m.n), "training output must hold n values");
-    c.make_current();
-    m.y = DevBuf<double>(c, m.n_pad);
-    m.alpha = DevBuf<double>(c, m.n_pad);
-    DevBuf<double> work(c, m.n_pad);
-    k::fill(c.main, m.y.get(), m.n_pad, 0.0);
-    upload(c, m.y.get(), y, static_cast<std::size_t>(m.n));
-    solve_spd(c, m.L.get(), m.lda, m.Winv.get(), m.n_pad, m.y.get(), work.get(), m.alpha.get(), m.Wpanel.get(), m.wblock);
-    if (m.precision == GPRAT_PRECISION_MIXED)
-        refine_alpha(m, work.get());
-    c.sync();
-}
-
 void fit(Context &c,
          Model &m,
          const double *x,
@@ -1200,8 +1251,37 @@ void fit(Context &c,
          int precision)
 {
     require(y != nullptr && y_len >= static_cast<std::size_t>(n), "training output must hold n values");
-    factor(c, m, x, x_len, n, r, theta, precision);
-    attach_targets(m, y, y_len);
+    check_training(x, x_len, n, r, theta, precision);
+    const bool mixed = precision == GPRAT_PRECISION_MIXED;
+    const int n_pad = static_cast<int>(padded(n));
+    c.make_current();
+    m.y = DevBuf<double>(c, n_pad);
+    k::fill(c.main, m.y.get(), n_pad, 0.0);
+    upload(c, m.y.get(), y, static_cast<std::size_t>(n));
+    DevBuf<double> rhs;
+    if (one_launch(n_pad, mixed))
+    {
+        // the targets ride along as a row below the matrix: z = L^-1 y
+        rhs = DevBuf<double>(c, static_cast<std::size_t>(64) * leading_dim(n_pad));
+        GP_HIP(hipMemcpyAsync(rhs.get(), m.y.get(), sizeof(double) * n_pad, hipMemcpyDeviceToDevice, c.main));
+    }
+    factor(c, m, x, x_len, n, r, theta, precision, rhs.get());
+    m.alpha = DevBuf<double>(c, n_pad);
+    DevBuf<double> work(c, n_pad);
+    if (rhs.get())
+    {
+        Timed t(c, c.main, "solve");
+        solve_upper(c, m.L.get(), m.lda, n_pad, rhs.get(), m.alpha.get(), m.Wpanel.get(), m.wblock);
+    }
+    else
+        solve_spd(c, m.L.get(), m.lda, m.Winv.get(), n_pad, m.y.get(), work.get(), m.alpha.get(), m.Wpanel.get(), m.wblock);
+    c.sync();
+    check_pivots(c);
+    if (mixed)
+    {
+        refine_alpha(m, work.get());
+        c.sync();
+    }
 }
 
 void predict_view(const FactorView &m, const double *z, std::size_t z_len, int mt, double *mean, double *var)
@@ -1405,8 +1485,6 @@ void predict_with_uncertainty_once(Context &c, const double *x, std::size_t x_le
     m.x = DevBuf<double>(c, xl);
     m.L = DevBuf<double>(c, (static_cast<std::size_t>(m.n_pad) + extra) * m.lda);
     m.Winv = DevBuf<double>(c, static_cast<std::size_t>(m.n_pad) * 64);
-    m.wblock = panel_width(m.n_pad);
-    m.Wpanel = DevBuf<double>(c, static_cast<std::size_t>(ceil_div(m.n_pad, m.wblock)) * m.wblock * m.wblock);
     DevBuf<double> dz(c, zl);
     upload(c, m.x.get(), x, xl);
     upload(c, dz.get(), z, zl);
@@ -1422,7 +1500,7 @@ void predict_with_uncertainty_once(Context &c, const double *x, std::size_t x_le
     // the rows below K come out as K* L^-T (test row t: v_t = L^-1 k_t) and
     // (L^-1 y)^T, so the mean is K* K^-1 y = V (L^-1 y) and the variance
     // v - |v_t|^2: no alpha and no separate solve
-    cholesky(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), false, m.Wpanel.get(), extra);
+    cholesky(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), false, nullptr, extra);
     DevBuf<double> dmean(c, mt), colsq(c, mt), dvar(c, mt);
     {
         Timed t(c, c.main, "mean");
@@ -1436,6 +1514,7 @@ void predict_with_uncertainty_once(Context &c, const double *x, std::size_t x_le
     GP_HIP(hipMemcpyAsync(mean, dmean.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
     GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
     c.sync();
+    check_pivots(c);
 }
 
 FactorView view(const Model &m)
@@ -1681,6 +1760,7 @@ void cholesky_tiles(Model &m, int T, int b, double *out)
     k::gather_tiles(c.main, m.L.get(), m.lda, m.x.get(), m.r, m.sek, T, b, d.get());
     GP_HIP(hipMemcpyAsync(out, d.get(), count * sizeof(double), hipMemcpyDefault, c.main));
     c.sync();
+    check_pivots(c);
 }
 
 }  // namespace gpamd

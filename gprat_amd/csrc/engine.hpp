@@ -128,6 +128,7 @@ struct Context
     std::recursive_mutex mu;
 
     DevBuf<int> info;         // smallest non-positive pivot column
+    int *host_info = nullptr; // its pinned copy (check_pivots)
     DevBuf<double> scalars;   // reduction results
 
     // profiling
@@ -267,16 +268,27 @@ void cholesky_fp64(Context &c, double *A, long lda, int n_pad, double *Winv);
 // extra: rows below the n_pad x n_pad matrix (A holds n_pad + extra rows)
 // that the factorisation treats as rows of L below it: on return they hold
 // B L^-T for the B they held (the forward solve of their transposes).
-void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel = nullptr, int extra = 0);
+// Their rows start at X (row stride lda; null: right below A). The factor is
+// complete in stream order on c.main; c.sync() and check_pivots() report a
+// pivot that was not positive.
+void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel = nullptr, int extra = 0, double *X = nullptr);
+// After cholesky() and a c.sync(): throws GPRAT_ERR_NOT_SPD if a pivot was
+// not positive.
+void check_pivots(Context &c);
 int panel_width(int n_pad);
+// The factorisation of this size runs as one dataflow launch (k_flow.hip).
+bool one_launch(int n_pad, bool mixed);
 void refine_alpha(Model &m, double *work);
 void solve_spd(Context &c, const double *L, long lda, const double *Winv, int n_pad, const double *y, double *work, double *out,
                const double *Wpanel = nullptr, int wblock = 0);
 void trsm_blocked(Context &c, const double *L, long lda, const double *Winv, const double *Wpanel, int wblock, int n_pad, double *B,
                   long ldb, int ncols, bool tri_rhs, double *out, long ldo);
 
-void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int r, const double theta[3], int precision);
-void attach_targets(Model &m, const double *y, std::size_t y_len);
+// rhs: a block row (64 x m.lda) that rides along and leaves as rhs L^-T
+// (one_launch() sizes only). keep_inverses: the panels' whole inverses, which
+// the solves step through, are wanted. Pivots as cholesky().
+void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int r, const double theta[3], int precision,
+            double *rhs = nullptr, bool keep_inverses = true);
 void fit(Context &c,
          Model &m,
          const double *x,

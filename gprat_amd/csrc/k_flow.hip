@@ -1,0 +1,546 @@
+// Cholesky factorisation as one launch: 64x64 tiles as a dataflow.
+//
+// The launch-per-step schedule pays two launches and their gaps for each 64
+// columns of the diagonal-block chain; below some ten thousand columns that
+// chain, not the matrix cores, sets the time. Here workgroups take tasks from
+// a device counter and wait for the tiles they need on progress counters, so a
+// step of the chain costs a factor, two block products and one hand-over
+// between workgroups.
+//
+// Block columns come in panels of PANEL. A tile of panel p is left-looking
+// over panels p - 1 and p (acc = sum_k L_ik L_jk^T in registers, at most
+// 2 PANEL - 1 products, then L_ij = (A_ij - acc) W_jj^T); panels 0 .. p - 2
+// have been subtracted from A_ij before, one update task each. Task order: the
+// first diagonal block, then per block column j of panel p
+//  * the pair L(j+1, j) and the diagonal block j + 1 (one task: the chain),
+//    the tiles (i, j) below it, and column j of the rows that ride along
+//    below the matrix (right-hand sides: they leave as B L^-T);
+//  * a PANEL-th of panel p - 1's updates of the tiles right of panel p,
+//    nearest columns first: they fill the device while the chain runs.
+// Every task depends only on tasks with smaller numbers, which have been
+// taken by running workgroups, so every wait ends whatever else holds the
+// device; a spin limit turns a lost update into an error instead of a hang.
+//
+// progress[r] counts the finished tiles of row r from its first one on (L_rr
+// counts too): a tile needs progress[i] > k and progress[j] > k for its k-th
+// product and progress[j] > j for W_jj. applied[r][c] counts the panels
+// subtracted from tile (r, c). Results are written with ordinary stores, made
+// visible by an agent-scope release before the counter moves, and read after
+// an agent-scope acquire.
+//
+// Measured on MI355X: a step of the chain takes 14.5 us when nothing else runs
+// (factor 8, the two products 2.9, stores and hand-over 2.5), 25 to 40 us
+// beside a full device; n = 1024 / 2048 / 4992 / 8192 factored in 0.26 / 0.67 /
+// 2.2 / 5.8 ms (panel schedule: 0.70 / 1.5 / 4.1 / 8.6), the last at 32 TF/s:
+// a 64x64 tile's products read 64 KB of operands for 0.5 MFLOP.
+#include <algorithm>
+#include <climits>
+
+#include "block64.hpp"
+#include "block_mfma.hpp"
+#include "kernels.hpp"
+
+namespace gpamd::k
+{
+namespace
+{
+
+struct FlowArgs
+{
+    double *A;
+    long lda;
+    double *X;
+    int nb, ne, unit;
+    double *Winv;
+    int *info, *queue, *progress, *applied;
+    int tasks;
+};
+
+constexpr int NB = 64;
+constexpr int THREADS = 256;
+constexpr int PANEL = FLOW_PANEL;
+// polls before a wait gives up, and how often it looks whether another has
+// (a poll takes of the order of a microsecond: more than ten seconds)
+constexpr int SPIN_LIMIT = 1 << 24;
+constexpr int SPIN_LOOK = 1 << 10;
+
+__global__ __launch_bounds__(THREADS) void k_flow_init(FlowArgs a, long counters)
+{
+    const long i = static_cast<long>(blockIdx.x) * THREADS + threadIdx.x;
+    if (i == 0)
+        *a.info = INT_MAX;
+    if (i < counters)
+        a.queue[i] = 0;  // the queue, progress and applied counters lie one after another
+}
+
+__device__ __forceinline__ int load_counter(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+
+// Waits until counters p and q have reached `need`, and r `need_r`; returns the
+// smaller of p and q (at least `need`). Everything the counted tasks wrote is
+// then visible to the workgroup. words: two alternating result words in LDS.
+__device__ __forceinline__ int wait_for(const FlowArgs &a, const int *p, const int *q, int need, const int *r, int need_r, int *words, int &turn)
+{
+    int *word = words + (turn & 1);
+    turn++;
+    if (threadIdx.x == 0)
+    {
+        int v = min(load_counter(p), load_counter(q)), u = load_counter(r);
+        for (int spins = 1; v < need || u < need_r; spins++)
+        {
+            if (spins >= SPIN_LIMIT)
+                atomicMin(a.info, FLOW_STALLED);
+            if (spins % SPIN_LOOK == 0 && load_counter(a.info) == FLOW_STALLED)
+            {
+                v = max(v, need);
+                break;
+            }
+            // several columns away: poll seldom, so that hundreds of waiting
+            // workgroups leave the counters' cache lines to the chain
+            if (v < need - 1)
+                __builtin_amdgcn_s_sleep(64);
+            else
+                __builtin_amdgcn_s_sleep(2);
+            v = min(load_counter(p), load_counter(q));
+            u = load_counter(r);
+        }
+        *word = v;
+    }
+    __syncthreads();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    return *word;
+}
+
+__device__ __forceinline__ int wait_for(const FlowArgs &a, const int *p, const int *q, int need, int *words, int &turn)
+{
+    return wait_for(a, p, q, need, p, 0, words, turn);
+}
+
+// This workgroup's stores are visible to whoever sees the counter at
+// `value`: every wavefront's have reached the L2 at the barrier, and the
+// release writes the L2 back.
+__device__ __forceinline__ void publish(int *p, int value)
+{
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0)
+        __hip_atomic_store(p, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// acc += A A^T beside mfma_nt_acc's A B^T, from the same staged rows.
+__device__ __forceinline__ void mfma_pair(const double *A, const double *B, blk::v4d (&ab)[2][2], blk::v4d (&aa)[2][2], int tid)
+{
+    const int lane = tid & 63, w = tid >> 6;
+    const int lm = lane & 15, lk = lane >> 4;
+    const int r0 = (w >> 1) * 32, c0 = (w & 1) * 32;
+#pragma unroll 4
+    for (int k0 = 0; k0 < NB; k0 += 4)
+    {
+        double a[2], b[2], t[2];
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+        {
+            a[i] = A[(r0 + i * 16 + lm) * blk::XS + k0 + lk];
+            b[i] = B[(c0 + i * 16 + lm) * blk::XS + k0 + lk];
+            t[i] = A[(c0 + i * 16 + lm) * blk::XS + k0 + lk];
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+            {
+                ab[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], ab[i][j], 0, 0, 0);
+                aa[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], t[j], aa[i][j], 0, 0, 0);
+            }
+    }
+}
+
+// Block products k0 .. k1 - 1 of two block rows through the LDS stages, the
+// next pair of blocks on its way while the current one is multiplied.
+template <class F>
+__device__ __forceinline__ void stream_blocks(const double *ri, const double *rj, long lda, int k0, int k1, double *buf0, double *buf1, int tid, F product)
+{
+    blk::d2 va[8], vb[8];
+    blk::load_block(ri + static_cast<long>(NB) * k0, lda, va, tid);
+    blk::load_block(rj + static_cast<long>(NB) * k0, lda, vb, tid);
+    for (int k = k0; k < k1; k++)
+    {
+        __syncthreads();  // every wavefront is done with the previous pair
+        blk::store_block(buf0, va, tid);
+        blk::store_block(buf1, vb, tid);
+        __syncthreads();
+        if (k + 1 < k1)
+        {
+            blk::load_block(ri + static_cast<long>(NB) * (k + 1), lda, va, tid);
+            blk::load_block(rj + static_cast<long>(NB) * (k + 1), lda, vb, tid);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        product();
+    }
+}
+
+// buf[r][c] (stride XS) = s - acc at this lane's accumulator positions.
+__device__ __forceinline__ void stage_difference(double *buf, const double (&s)[16], const blk::v4d (&acc)[2][2], int tid)
+{
+    int q = 0;
+    blk::for_each(acc, [&](int r, int c, double v) { buf[r * blk::XS + c] = s[q++] - v; }, tid);
+}
+
+// The thread's index, hidden from the compiler: what follows from it is not
+// carried from task to task (the addresses of a task's block operations, kept
+// across the task loop, overflowed the registers).
+__device__ __forceinline__ int own_thread()
+{
+    int t = threadIdx.x;
+    asm volatile("" : "+v"(t));
+    return t;
+}
+
+__device__ __forceinline__ double *row_of(const FlowArgs &a, int i)
+{
+    return i < a.nb ? a.A + static_cast<long>(NB) * i * a.lda : a.X + static_cast<long>(NB) * (i - a.nb) * a.lda;
+}
+__device__ __forceinline__ int *applied_of(const FlowArgs &a, int i, int j) { return a.applied + static_cast<long>(i) * a.nb + j; }
+
+// L = S W^T for W lower triangular (buf S and W staged, stride XS): wavefront
+// w owns rows 16 w .. 16 w + 15, column block c needs k < 16 (c + 1) only.
+__device__ __forceinline__ void solve_product(const double *S, const double *W, blk::v4d (&acc)[4], int tid)
+{
+    const int lane = tid & 63, w = tid >> 6;
+    const int lm = lane & 15, lk = lane >> 4;
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+        acc[c] = blk::v4d{ 0.0, 0.0, 0.0, 0.0 };
+#pragma unroll
+    for (int kc = 0; kc < 4; kc++)
+#pragma unroll
+        for (int k0 = 16 * kc; k0 < 16 * kc + 16; k0 += 4)
+        {
+            const double a = S[(16 * w + lm) * blk::XS + k0 + lk];
+#pragma unroll
+            for (int c = kc; c < 4; c++)
+                acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, W[(16 * c + lm) * blk::XS + k0 + lk], acc[c], 0, 0, 0);
+        }
+}
+
+// f(row, column, value) over a solve_product's results.
+template <class F>
+__device__ __forceinline__ void for_each_solved(const blk::v4d (&acc)[4], int tid, F f)
+{
+    const int lane = tid & 63, w = tid >> 6;
+    const int lm = lane & 15, lk = lane >> 4;
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            f(16 * w + lk + 4 * e, 16 * c + lm, acc[c][e]);
+}
+
+// D -= L L^T for D and L staged (stride XS), the ten 16x16 tiles on and below
+// the diagonal dealt to the four wavefronts (3, 3, 2, 2).
+__device__ __forceinline__ void subtract_square(double *D, const double *L, int tid)
+{
+    const int lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int lm = lane & 15, lk = lane >> 4;
+    constexpr int rows[4][3] = { { 0, 3, 3 }, { 1, 3, 3 }, { 1, 2, -1 }, { 2, 2, -1 } };
+    constexpr int cols[4][3] = { { 0, 0, 1 }, { 0, 2, 3 }, { 1, 0, -1 }, { 1, 2, -1 } };
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+    {
+        if (w != v)
+            continue;
+        blk::v4d acc[3];
+        double d[3][4];
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+            if (rows[v][t] >= 0)
+            {
+                acc[t] = blk::v4d{ 0.0, 0.0, 0.0, 0.0 };
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    d[t][e] = D[(16 * rows[v][t] + lk + 4 * e) * blk::XS + 16 * cols[v][t] + lm];
+            }
+#pragma unroll
+        for (int k0 = 0; k0 < NB; k0 += 4)
+#pragma unroll
+            for (int t = 0; t < 3; t++)
+                if (rows[v][t] >= 0)
+                    acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(L[(16 * rows[v][t] + lm) * blk::XS + k0 + lk],
+                                                                  L[(16 * cols[v][t] + lm) * blk::XS + k0 + lk], acc[t], 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 3; t++)
+            if (rows[v][t] >= 0)
+            {
+#pragma unroll
+                for (int e = 0; e < 4; e++)
+                    D[(16 * rows[v][t] + lk + 4 * e) * blk::XS + 16 * cols[v][t] + lm] = d[t][e] - acc[t][e];
+            }
+    }
+}
+
+typedef __attribute__((address_space(3))) double lds_double;
+
+// Out of line: the elimination's registers stay out of the tasks' allocation.
+__device__ __noinline__ void factor_staged(lds_double *d, lds_double *w, int *info, int col0)
+{
+    factor_block64(reinterpret_cast<double(*)[blk::XS]>((double *)d), reinterpret_cast<double(*)[blk::XS]>((double *)w), info, col0);
+}
+
+// The columns' panels start their products here (see above).
+__device__ __forceinline__ int first_product(int column) { return max(0, (column / PANEL - 1) * PANEL); }
+
+// L(j+1, j) and the diagonal block j + 1 (q = j + 1 >= 1), or block 0: the
+// chain, at a raised wave priority beside the other tasks of its CU.
+__device__ __forceinline__ void diagonal_task(const FlowArgs &a, int q, double *buf0, double *buf1, int *words, int &turn)
+{
+    const int tid = own_thread();
+    double *rq = row_of(a, q);
+    double *dst = rq + static_cast<long>(NB) * q;
+    double d[16];
+    __builtin_amdgcn_s_setprio(2);
+    if (q == 0)
+        blk::load_at_acc(dst, a.lda, d, tid);
+    else
+    {
+        const int j = q - 1;
+        const double *rj = row_of(a, j);
+        blk::v4d off[2][2], dia[2][2];
+        blk::zero(off);
+        blk::zero(dia);
+        const int pair = first_product(q);  // both tiles' products from here on
+        for (int k = first_product(j); k < j;)
+        {
+            const int k1 = min(k < pair ? min(j, pair) : j, wait_for(a, a.progress + q, a.progress + j, k + 1, words, turn));
+            if (k < pair)
+                stream_blocks(rq, rj, a.lda, k, k1, buf0, buf1, tid, [&] { blk::mfma_nt_acc(buf0, buf1, off, tid); });
+            else
+                stream_blocks(rq, rj, a.lda, k, k1, buf0, buf1, tid, [&] { mfma_pair(buf0, buf1, off, dia, tid); });
+            k = k1;
+        }
+        double *lqj = rq + static_cast<long>(NB) * j;
+        if (q / PANEL >= 2)
+            wait_for(a, applied_of(a, q, q), applied_of(a, q, q), q / PANEL - 1, applied_of(a, q, j), j / PANEL - 1, words, turn);
+        double s[16];
+        blk::load_at_acc(lqj, a.lda, s, tid);
+        blk::load_at_acc(dst, a.lda, d, tid);
+        __syncthreads();
+        stage_difference(buf0, s, off, tid);
+        int e = 0;
+        blk::for_each(dia, [&](int, int, double v) { d[e++] -= v; }, tid);
+        wait_for(a, a.progress + j, a.progress + j, j + 1, words, turn);
+        blk::stage_block(buf1, a.Winv + static_cast<long>(j) * NB * NB, NB, tid);
+        __syncthreads();
+        blk::v4d l[4];
+        solve_product(buf0, buf1, l, tid);
+        __syncthreads();
+        for_each_solved(l, tid,
+                        [&](int r, int c, double v)
+                        {
+                            buf0[r * blk::XS + c] = v;
+                            lqj[static_cast<long>(r) * a.lda + c] = v;
+                        });
+    }
+    blk::v4d pos[2][2];
+    int e = 0;
+    blk::for_each(pos, [&](int r, int c, double) { buf1[r * blk::XS + c] = c <= r ? d[e] : 0.0; e++; }, tid);
+    __syncthreads();
+    if (q > 0)
+    {
+        subtract_square(buf1, buf0, tid);
+        publish(a.progress + q, q);  // its barrier: the differences are in place
+    }
+    factor_staged((lds_double *)buf1, (lds_double *)buf0, a.info, NB * q);
+    // the inverse first: the next step waits for it, nothing in this launch for L_qq
+    double *w = a.Winv + static_cast<long>(q) * NB * NB;
+#pragma unroll
+    for (int s = 0; s < NB * NB / 2 / THREADS; s++)
+    {
+        const int t = tid + THREADS * s, r = t >> 5, c = (t & 31) * 2;
+        const blk::d2 v = *reinterpret_cast<const blk::d2 *>(buf0 + r * blk::XS + c);
+        *reinterpret_cast<blk::d2 *>(w + r * NB + c) = blk::d2{ c <= r ? v[0] : 0.0, c + 1 <= r ? v[1] : 0.0 };
+    }
+    publish(a.progress + q, q + 1);
+    __builtin_amdgcn_s_setprio(0);
+    for (int t = tid; t < NB * NB; t += THREADS)
+    {
+        const int r = t >> 6, c = t & 63;
+        if (c <= r)
+            dst[static_cast<long>(r) * a.lda + c] = buf1[r * blk::XS + c];
+    }
+}
+
+// Tile (i, j) off the diagonal. unit >= 0: a row that starts from the identity
+// in block column `unit`.
+__device__ __forceinline__ void off_task(const FlowArgs &a, int i, int j, int unit, double *buf0, double *buf1, int *words, int &turn)
+{
+    const int tid = own_thread();
+    double *ri = row_of(a, i);
+    const double *rj = row_of(a, j);
+    double *dst = ri + static_cast<long>(NB) * j;
+    blk::v4d acc[2][2];
+    blk::zero(acc);
+    const int before = j / PANEL - 1;                     // panels subtracted by update tasks
+    const bool stored = unit < 0 || unit / PANEL < before;  // the tile has a stored value
+    for (int k = max(first_product(j), unit); k < j;)
+    {
+        const int k1 = min(j, wait_for(a, a.progress + i, a.progress + j, k + 1, words, turn));
+        stream_blocks(ri, rj, a.lda, k, k1, buf0, buf1, tid, [&] { blk::mfma_nt_acc(buf0, buf1, acc, tid); });
+        k = k1;
+    }
+    double s[16];
+    if (stored)
+    {
+        if (before >= 1)
+            wait_for(a, applied_of(a, i, j), applied_of(a, i, j), before, words, turn);
+        blk::load_at_acc(dst, a.lda, s, tid);
+    }
+    else
+    {
+        int e = 0;
+        blk::for_each(acc, [&](int r, int c, double) { s[e++] = (j == unit && r == c) ? 1.0 : 0.0; }, tid);
+    }
+    __syncthreads();
+    stage_difference(buf0, s, acc, tid);
+    wait_for(a, a.progress + j, a.progress + j, j + 1, words, turn);
+    blk::stage_block(buf1, a.Winv + static_cast<long>(j) * NB * NB, NB, tid);
+    __syncthreads();
+    blk::v4d l[4];
+    solve_product(buf0, buf1, l, tid);
+    for_each_solved(l, tid, [&](int r, int c, double v) { dst[static_cast<long>(r) * a.lda + c] = v; });
+    publish(a.progress + i, j + 1);
+}
+
+// Tile (i, j) -= panel p's products.
+__device__ __forceinline__ void update_task(const FlowArgs &a, int i, int j, int p, int unit, double *buf0, double *buf1, int *words, int &turn)
+{
+    const int tid = own_thread();
+    double *dst = row_of(a, i) + static_cast<long>(NB) * j;
+    const int k0 = max(p * PANEL, unit), k1 = (p + 1) * PANEL;
+    const bool stored = unit < 0 || unit / PANEL < p;
+    blk::v4d acc[2][2];
+    blk::zero(acc);
+    wait_for(a, a.progress + i, a.progress + j, k1, applied_of(a, i, j), stored ? p : 0, words, turn);
+    stream_blocks(row_of(a, i), row_of(a, j), a.lda, k0, k1, buf0, buf1, tid, [&] { blk::mfma_nt_acc(buf0, buf1, acc, tid); });
+    double s[16];
+    if (stored)
+        blk::load_at_acc(dst, a.lda, s, tid);
+    else
+    {
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+            s[e] = 0.0;
+    }
+    int e = 0;
+    blk::for_each(acc, [&](int r, int c, double v) { dst[static_cast<long>(r) * a.lda + c] = s[e++] - v; }, tid);
+    publish(applied_of(a, i, j), p + 1);
+}
+
+// Rows below the matrix that panel p's updates of later columns reach.
+__host__ __device__ __forceinline__ int updated_extra(int ne, int unit, int p)
+{
+    const int reach = (p + 1) * PANEL;
+    return unit && reach < ne ? reach : ne;
+}
+
+// Tasks of block column j: its tiles and its share of panel j / PANEL - 1's
+// updates [*u0, *u0 + *updates).
+__host__ __device__ __forceinline__ int column_tiles(int nb, int ne, int unit, int j) { return (nb - 1 - j) + (unit && j + 1 < ne ? j + 1 : ne); }
+__host__ __device__ __forceinline__ void column_updates(int nb, int ne, int unit, int j, long *u0, int *updates)
+{
+    const int p = j / PANEL - 1, m = nb - (p + 2) * PANEL;
+    *u0 = 0;
+    *updates = 0;
+    if (p < 0 || m <= 0)
+        return;
+    const long all = static_cast<long>(m) * (m + 1) / 2 + static_cast<long>(m) * updated_extra(ne, unit, p);
+    const int c = j % PANEL;
+    // rounded up: the first tile, which the next panel's first diagonal
+    // block needs, is in the first share
+    const long lo = (all * c + PANEL - 1) / PANEL, hi = (all * (c + 1) + PANEL - 1) / PANEL;
+    *u0 = lo;
+    *updates = static_cast<int>(hi - lo);
+}
+
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_flow(FlowArgs a)
+{
+    __shared__ alignas(16) double buf0[NB * blk::XS];
+    __shared__ alignas(16) double buf1[NB * blk::XS];
+    __shared__ int words[2];
+    __shared__ int next;
+    int turn = 0;
+    int j = 0, first = 1;  // the current column and its first task's number
+    long u0 = 0;
+    int updates = 0, tiles = column_tiles(a.nb, a.ne, a.unit, 0);
+    for (;;)
+    {
+        __syncthreads();  // the previous task's LDS reads are done
+        if (threadIdx.x == 0)
+            next = atomicAdd(a.queue, 1);
+        __syncthreads();
+        const int t = __builtin_amdgcn_readfirstlane(next);
+        if (t >= a.tasks)
+            return;
+        if (t == 0)
+        {
+            diagonal_task(a, 0, buf0, buf1, words, turn);
+            continue;
+        }
+        // task numbers only grow: the walk is incremental
+        while (t >= first + tiles + updates)
+        {
+            first += tiles + updates;
+            j++;
+            tiles = column_tiles(a.nb, a.ne, a.unit, j);
+            column_updates(a.nb, a.ne, a.unit, j, &u0, &updates);
+        }
+        const int idx = t - first, below = a.nb - 1 - j;
+        if (below > 0 && idx == 0)
+            diagonal_task(a, j + 1, buf0, buf1, words, turn);
+        else if (idx < below)
+            off_task(a, j + 1 + idx, j, -1, buf0, buf1, words, turn);
+        else if (idx < tiles)
+            off_task(a, a.nb + idx - below, j, a.unit ? idx - below : -1, buf0, buf1, words, turn);
+        else
+        {
+            const int p = j / PANEL - 1, extra = updated_extra(a.ne, a.unit, p);
+            long u = u0 + (idx - tiles);
+            int c = (p + 2) * PANEL;
+            while (u >= (a.nb - c) + extra)
+                u -= (a.nb - c++) + extra;
+            const int r = static_cast<int>(u), own = a.nb - c;
+            update_task(a, r < own ? c + r : a.nb + r - own, c, p, a.unit && r >= own ? r - own : -1, buf0, buf1, words, turn);
+        }
+    }
+}
+
+}  // namespace
+
+long flow_counters(int nb, int ne) { return 1 + (static_cast<long>(nb) + ne) * (1 + nb); }
+
+void flow_cholesky(hipStream_t s, const FlowCall &f, int cus)
+{
+    require(f.nb >= 1 && f.ne >= 0 && f.lda % 2 == 0 && f.lda >= static_cast<long>(NB) * f.nb, "flow_cholesky: bad shape");
+    require(!f.unit || f.ne <= f.nb, "flow_cholesky: more unit rows than columns");
+    require(f.ne == 0 || (f.X != nullptr && reinterpret_cast<uintptr_t>(f.X) % 16 == 0), "flow_cholesky: bad rows below the matrix");
+    require(reinterpret_cast<uintptr_t>(f.A) % 16 == 0 && reinterpret_cast<uintptr_t>(f.Winv) % 16 == 0,
+            "flow_cholesky: operands must be 16-byte aligned");
+    long tasks = 1;
+    for (int j = 0; j < f.nb; j++)
+    {
+        long u0;
+        int updates;
+        column_updates(f.nb, f.ne, f.unit, j, &u0, &updates);
+        tasks += column_tiles(f.nb, f.ne, f.unit, j) + updates;
+    }
+    // every running workgroup may add one number past the last task
+    require(tasks < (1L << 30), "flow_cholesky: too many tiles");
+    const long counters = flow_counters(f.nb, f.ne);
+    const FlowArgs a{ f.A, f.lda, f.X, f.nb, f.ne, f.unit ? 1 : 0, f.Winv, f.info, f.counters, f.counters + 1, f.counters + 1 + f.nb + f.ne,
+                      static_cast<int>(tasks) };
+    hipLaunchKernelGGL(k_flow_init, dim3(static_cast<unsigned>(ceil_div(counters, THREADS))), dim3(THREADS), 0, s, a, counters);
+    GP_CHECK_LAUNCH();
+    const long wgs = std::min<long>(tasks, 2L * cus);  // two workgroups' LDS fit a CU
+    hipLaunchKernelGGL(k_flow, dim3(static_cast<unsigned>(wgs)), dim3(THREADS), 0, s, a);
+    GP_CHECK_LAUNCH();
+}
+
+}  // namespace gpamd::k

@@ -260,6 +260,53 @@ __global__ __launch_bounds__(THREADS) void k_panel_tasks(PanelArgs a)
     }
 }
 
+// One panel's arguments for the inverse tasks run over all panels at once.
+struct InverseArgs
+{
+    const double *L;
+    long lda;
+    const double *Winv;
+    int n, width;
+    double *Wb, *tmp;
+};
+
+__device__ __forceinline__ PanelArgs panel_of(const InverseArgs &g, int panel)
+{
+    PanelArgs a{};
+    a.h.A = const_cast<double *>(g.L);  // read only by these tasks
+    a.h.lda = g.lda;
+    a.h.p0 = static_cast<long>(panel) * g.width;
+    a.h.nb = min(g.width, static_cast<int>(g.n - a.h.p0)) / NB;
+    a.h.Winv = const_cast<double *>(g.Winv);
+    a.h.Wb = g.Wb + static_cast<long>(panel) * g.width * g.width;
+    a.h.ldw = g.width;
+    a.h.tmp = g.tmp;
+    return a;
+}
+
+__global__ __launch_bounds__(THREADS) void k_inverse_place(InverseArgs g)
+{
+    __shared__ alignas(16) double buf0[NB * blk::XS];
+    const int per = g.width / NB;
+    task_place(panel_of(g, blockIdx.x / per), blockIdx.x % per, buf0);
+}
+
+// Doubling level h of every panel (grid: block (rb, cb) of the pair, pair,
+// panel): the whole join at h = 1, one of its two phases above.
+__global__ __launch_bounds__(THREADS) void k_inverse_join(InverseArgs g, int h, int phase)
+{
+    __shared__ alignas(16) double buf0[NB * blk::XS];
+    __shared__ alignas(16) double buf1[NB * blk::XS];
+    const PanelArgs a = panel_of(g, blockIdx.z);
+    const int pair = blockIdx.y, rb = blockIdx.x / h, cb = blockIdx.x % h;
+    if (2 * h * pair + h + rb >= a.h.nb)
+        return;
+    if (h == 1)
+        task_joinf(a, 2 * pair, buf0, buf1);
+    else
+        task_join(a, phase, h, pair, rb, cb, (blockIdx.z * gridDim.y + pair) * h * h, buf0, buf1);
+}
+
 // Panel rows below a factored diagonal block: X = A W^T for the R rows at
 // r0 of the panel's columns [p0, p0 + 64 nbw), W the block's k-major
 // inverse (lower: X(i, c) = sum_{t <= c} A(i, t) W(c, t)^T over 64x64
@@ -881,6 +928,39 @@ void leaf_solve(hipStream_t s, const double *Wk, long ldw, int rows, const doubl
     require((nbr + 1) / 2 <= 65535, "leaf_solve: too many rows for one launch");
     hipLaunchKernelGGL(k_leaf_solve, dim3(cols / NB, (nbr + 1) / 2), dim3(THREADS), 0, s, Wk, ldw, nbr, B, ldb, V, ldv);
     GP_CHECK_LAUNCH();
+}
+
+// pairs of doubling level h in a panel of `per` blocks
+static int inverse_pairs(int per, int h) { return static_cast<int>(ceil_div(per - h, 2L * h)); }
+
+long panel_inverses_scratch(int n, int width)
+{
+    const int per = width / NB, panels = static_cast<int>(ceil_div(n, width));
+    long most = 0;
+    for (int h = 2; h < per; h *= 2)
+        most = std::max(most, static_cast<long>(panels) * inverse_pairs(per, h) * h * h * NB * NB);
+    return most;
+}
+
+void panel_inverses(hipStream_t s, const double *L, long lda, const double *Winv, int n, int width, double *Wb, double *tmp)
+{
+    require(n > 0 && n % NB == 0 && width > 0 && width % NB == 0 && lda % 2 == 0 && lda >= n, "panel_inverses: bad shape");
+    require(reinterpret_cast<uintptr_t>(L) % 16 == 0 && reinterpret_cast<uintptr_t>(Winv) % 16 == 0 && reinterpret_cast<uintptr_t>(Wb) % 16 == 0
+                && reinterpret_cast<uintptr_t>(tmp) % 16 == 0,
+            "panel_inverses: operands must be 16-byte aligned");
+    const int per = width / NB;
+    const unsigned panels = static_cast<unsigned>(ceil_div(n, width));
+    require(panels <= 65535, "panel_inverses: too many panels");
+    const InverseArgs g{ L, lda, Winv, n, width, Wb, tmp };
+    hipLaunchKernelGGL(k_inverse_place, dim3(static_cast<unsigned>(n / NB)), dim3(THREADS), 0, s, g);
+    GP_CHECK_LAUNCH();
+    for (int h = 1; h < per; h *= 2)
+        for (int phase = 0; phase < (h == 1 ? 1 : 2); phase++)
+        {
+            hipLaunchKernelGGL(k_inverse_join, dim3(static_cast<unsigned>(h) * h, static_cast<unsigned>(inverse_pairs(per, h)), panels), dim3(THREADS),
+                               0, s, g, h, phase);
+            GP_CHECK_LAUNCH();
+        }
 }
 
 void solve_lower_step(hipStream_t s, const double *L, long lda, const double *Winv, double *rhs, double *out, int n_pad, int j)

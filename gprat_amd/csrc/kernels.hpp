@@ -282,6 +282,42 @@ void rows_solve(hipStream_t s, const double *A, long lda, long r0, long p0, int 
 // x cols. rows and cols are multiples of 64.
 void leaf_solve(hipStream_t s, const double *Wk, long ldw, int rows, const double *B, long ldb, int cols, double *V, long ldv);
 
+// Whole inverses of the `width`-wide diagonal blocks of L (n x n, n a
+// multiple of 64; the last block may be narrower) from the row-major inverses
+// Winv of its 64x64 diagonal blocks: block b k-major (W(r, c) at [c * width +
+// r], zero above the diagonal) at Wb + b * width^2. tmp:
+// panel_inverses_scratch(n, width) doubles.
+long panel_inverses_scratch(int n, int width);
+void panel_inverses(hipStream_t s, const double *L, long lda, const double *Winv, int n, int width, double *Wb, double *tmp);
+
+// ---- factorisation as one dataflow launch (k_flow.hip) -------------------
+
+// *info when a wait gave up (never a column).
+constexpr int FLOW_STALLED = -1;
+// 64-wide block columns per panel of the task order (k_flow.hip).
+constexpr int FLOW_PANEL = 8;
+// A: the lower triangle of an nb x nb matrix of 64x64 blocks (row stride
+// lda), factored in place. X: ne block rows of the same width and stride that
+// leave as X L^-T (rows are independent, so what unused ones hold does not
+// matter). unit: those rows start as the identity's first ne block rows
+// instead (X is not read; the blocks left of a row's first nonzero one are not
+// written). The row-major inverses of L's 64x64 diagonal blocks
+// go to Winv. counters: flow_counters(nb, ne) ints; info: the smallest
+// non-positive pivot's column, INT_MAX or FLOW_STALLED (both device memory,
+// set by the call). cus: the device's compute units.
+struct FlowCall
+{
+    double *A;
+    long lda;
+    double *X;
+    int nb, ne;
+    bool unit;
+    double *Winv;
+    int *info, *counters;
+};
+long flow_counters(int nb, int ne);
+void flow_cholesky(hipStream_t s, const FlowCall &f, int cus);
+
 // Block steps of the vector solves with the saved diagonal-block inverses
 // Winv (block J at Winv + J*64*64). Forward: out[J] = W_JJ rhs[J],
 // rhs[later] -= L[later, J] out[J]; run J = 0 .. n_pad/64-1 in order.

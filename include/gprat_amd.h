@@ -57,7 +57,8 @@ enum
      * form k^T K^-1 k to second order; gprat_model_set_variance_refinement
      * switches that correction off (FP32 forward solve only). The loss's
      * log-determinant and the gradient's K^-1 come from the mixed-precision
-     * factor unrefined. */
+     * factor unrefined. Up to about ten thousand training points the whole
+     * factor is FP64: there the FP32 updates would not shorten the fit. */
     GPRAT_PRECISION_MIXED = 1
 };
 

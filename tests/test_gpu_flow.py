@@ -1,0 +1,99 @@
+"""The factorisation as one dataflow launch (gprat_amd/csrc/k_flow.hip) against
+the panel schedule at the sizes around its 64-wide tiles and its panels of
+eight (the tiled right-looking Cholesky of core/src/cpu/gp_algorithms.cpp)."""
+import os
+from contextlib import contextmanager
+
+import numpy as np
+import pytest
+
+from conftest import norm_rel
+from gprat_amd import capi, datagen
+
+pytestmark = pytest.mark.gpu
+
+# two Cholesky factors of one matrix agree to about n eps cond; cond <= (n v + noise) / noise
+# <= 4e4 here and n <= 2500: 2500 * 1.1e-16 * 4e4 = 1.1e-8 is the worst case, the errors
+# of the factor's entries are random: sqrt(n) in place of n, hence
+TOL = 2e-10
+
+
+@contextmanager
+def panel_schedule():
+    saved = os.environ.get("GPRAT_FLOW_LIMIT")
+    os.environ["GPRAT_FLOW_LIMIT"] = "0"
+    try:
+        yield
+    finally:
+        if saved is None:
+            del os.environ["GPRAT_FLOW_LIMIT"]
+        else:
+            os.environ["GPRAT_FLOW_LIMIT"] = saved
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = capi.Context(0, 1)
+    yield c
+    c.close()
+
+
+SIZES = [1, 64, 65, 500, 513, 1024, 1030, 1100, 1537, 2049, 2500]
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("m", [1, 70, 1000])
+def test_one_call(ctx, n, m):
+    x, y, z = datagen.gp_problem(n, m, 5)
+    args = (x, y, z, (1.0, 1.0, 0.1), 1, n, 1, m, 5)
+    mean, var = ctx.predict(*args, variance=True)
+    with panel_schedule():
+        pm, pv = ctx.predict(*args, variance=True)
+    assert norm_rel(mean, pm) < TOL and norm_rel(var, pv) < TOL
+
+
+@pytest.mark.parametrize("n", SIZES)
+@pytest.mark.parametrize("precision", [capi.PRECISION_FP64, capi.PRECISION_MIXED])
+def test_resident(ctx, n, precision):
+    x, y, z = datagen.gp_problem(n, 33, 8)
+    theta = (1.0, 1.0, 0.1)
+
+    def results(p):
+        m = ctx.fit(x, y, n, 8, theta, p)
+        out = (*m.predict(z, 33), m.loss(), m.gradient()[1])
+        m.release()
+        return out
+    got = results(precision)
+    with panel_schedule():
+        want = results(capi.PRECISION_FP64)
+    # the mixed model's variance is refined from FP32 solves: 1e-7 is its stated bar
+    for a, b, tol in zip(got, want, (TOL, TOL if precision == capi.PRECISION_FP64 else 1e-7, TOL, 10 * TOL)):
+        assert norm_rel(np.atleast_1d(a), np.atleast_1d(b)) < tol
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_tiles(ctx, n):
+    x, _, _ = datagen.gp_problem(n, 1, 8)
+    a = ctx.cholesky(x, (1.0, 1.0, 0.1), 1, n, 8)
+    with panel_schedule():
+        b = ctx.cholesky(x, (1.0, 1.0, 0.1), 1, n, 8)
+    assert norm_rel(a.ravel(), b.ravel()) < TOL
+
+
+def test_repeats_are_bit_identical(ctx):
+    x, y, z = datagen.gp_problem(1800, 300, 8)
+    args = (x, y, z, (1.0, 1.0, 0.1), 1, 1800, 1, 300, 8)
+    first = ctx.predict(*args, variance=True)
+    for _ in range(5):
+        again = ctx.predict(*args, variance=True)
+        assert np.array_equal(first[0], again[0]) and np.array_equal(first[1], again[1])
+
+
+@pytest.mark.parametrize("column", [70, 600, 1100, 1500])
+def test_first_failing_pivot(ctx, column):
+    n, r = 1600, 4
+    u = np.arange(n + r - 1) * 10.0
+    u[column:column + r] = u[:r]  # this window repeats the first one: its pivot is about 2 * noise < 0
+    with pytest.raises(capi.GpratError, match=f"at column {column}\\)"):
+        ctx.cholesky(u, (0.3, 1.0, -1e-3), 1, n, r)
+    assert ctx.cholesky(u, (0.3, 1.0, 1e-3), 1, n, r).shape == (1, n, n)
