@@ -270,7 +270,7 @@ int gprat_cholesky(gprat_context *ctx,
             gpamd::require(tiles_out != nullptr, "tiles_out is null");
             std::lock_guard<std::recursive_mutex> g(c.mu);
             gpamd::Model model;
-            gpamd::factor(c, model, train_in, train_in_len, t.n, n_reg, theta, GPRAT_PRECISION_FP64, nullptr, false);
+            gpamd::factor(c, model, train_in, train_in_len, t.n, n_reg, theta, GPRAT_PRECISION_FP64, {}, false);
             gpamd::cholesky_tiles(model, n_tiles, n_tile_size, tiles_out);
         });
 }

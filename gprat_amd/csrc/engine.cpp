@@ -485,12 +485,12 @@ void check_pivots(Context &c)
 
 // The factorisation as one launch, then the panels' whole inverses if they
 // are kept.
-static void flow(Context &c, double *A, long lda, int n_pad, double *Winv, double *Wpanel, double *X, int extra, bool unit = false)
+static void flow(Context &c, double *A, long lda, int n_pad, double *Winv, double *Wpanel, double *X, int extra, int unit)
 {
     Timed t(c, c.main, "cholesky");
     const int nb = n_pad / 64, ne = extra / 64;
     DevBuf<int> counters(c, static_cast<std::size_t>(k::flow_counters(nb, ne)));
-    k::flow_cholesky(c.main, k::FlowCall{ A, lda, X, nb, ne, unit, Winv, c.info.get(), counters.get() }, c.cus);
+    k::flow_cholesky(c.main, k::FlowCall{ A, lda, X, nb, ne, unit / 64, Winv, c.info.get(), counters.get() }, c.cus);
     if (Wpanel)
     {
         const int width = outer_block(n_pad);
@@ -504,16 +504,16 @@ void cholesky_fp64(Context &c, double *A, long lda, int n_pad, double *Winv) { c
 
 int panel_width(int n_pad) { return outer_block(n_pad); }
 
-void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel, int extra, double *X)
+void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel, int extra, double *X, int unit)
 {
     require(n_pad % 128 == 0 && lda >= n_pad && lda % 2 == 0, "cholesky: bad layout");
     require(extra >= 0 && extra % 64 == 0, "cholesky: extra rows must come in 64s");
     if (one_launch(n_pad, mixed))
     {
-        flow(c, A, lda, n_pad, Winv, Wpanel, X ? X : A + static_cast<long>(n_pad) * lda, extra);
+        flow(c, A, lda, n_pad, Winv, Wpanel, X ? X : A + static_cast<long>(n_pad) * lda, extra, unit);
         return;
     }
-    require(X == nullptr, "cholesky: the panel schedule takes its rows below the matrix");
+    require(X == nullptr && unit == 0, "cholesky: the panel schedule takes its rows below the matrix");
     // rows of L and the rows below it that ride along (right-hand sides)
     const long rows = static_cast<long>(n_pad) + extra;
     const bool ahead = use_lookahead() && c.panel != c.main;
@@ -1151,7 +1151,7 @@ static void check_training(const double *x, std::size_t x_len, int n, int r, con
     require(precision == GPRAT_PRECISION_FP64 || precision == GPRAT_PRECISION_MIXED, "unknown precision mode");
 }
 
-void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int r, const double theta[3], int precision, double *rhs,
+void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int r, const double theta[3], int precision, Riding riding,
             bool keep_inverses)
 {
     check_training(x, x_len, n, r, theta, precision);
@@ -1176,7 +1176,7 @@ void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int
         k::assemble_lower(c.main, m.x.get(), r, m.sek, m.L.get(), m.lda, n, m.n_pad);
     }
     cholesky(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), precision == GPRAT_PRECISION_MIXED, m.Wpanel.get(),
-             rhs ? 64 : 0, rhs);
+             riding.extra, riding.X, riding.unit);
     if (precision == GPRAT_PRECISION_MIXED)
     {
         // the covariance's strictly lower part, for the FP64 residual of the
@@ -1265,7 +1265,7 @@ void fit(Context &c,
         rhs = DevBuf<double>(c, static_cast<std::size_t>(64) * leading_dim(n_pad));
         GP_HIP(hipMemcpyAsync(rhs.get(), m.y.get(), sizeof(double) * n_pad, hipMemcpyDeviceToDevice, c.main));
     }
-    factor(c, m, x, x_len, n, r, theta, precision, rhs.get());
+    factor(c, m, x, x_len, n, r, theta, precision, { rhs.get(), rhs.get() ? 64 : 0, 0 });
     m.alpha = DevBuf<double>(c, n_pad);
     DevBuf<double> work(c, n_pad);
     if (rhs.get())
@@ -1636,6 +1636,8 @@ void batch_predict(Batch &b, int index, const double *z, std::size_t z_len, int 
                  z, z_len, mt, mean, var);
 }
 
+static double loss_of(const Model &m, const double *t);
+
 double loss(Model &m)
 {
     Context &c = *m.ctx;
@@ -1644,11 +1646,7 @@ double loss(Model &m)
     double t[3];
     GP_HIP(hipMemcpyAsync(t, c.scalars.get(), sizeof t, hipMemcpyDefault, c.main));
     c.sync();
-    // core/src/cpu/gp_optimizer.cpp:205-218
-    const double Nn = static_cast<double>(m.n);
-    double l = t[0] + t[1];
-    l += Nn * std::log(2.0 * std::numbers::pi);
-    return 0.5 * l / Nn;
+    return loss_of(m, t);
 }
 
 // Softplus chain factors, as core/src/cpu/gp_optimizer.cpp:12-36.
@@ -1658,12 +1656,35 @@ static double to_unconstrained(double p, bool noise)
 }
 static double sigmoid(double p) { return 1.0 / (1.0 + std::exp(-p)); }
 
+// The loss from its terms t (k::loss_terms), and the trainable gradient
+// entries from k::gradient_sums()' sums (core/src/cpu/gp_optimizer.cpp:205-225,
+// tiled_algorithms.cpp:413-426).
+static double loss_of(const Model &m, const double *t)
+{
+    const double Nn = static_cast<double>(m.n);
+    double l = t[0] + t[1];
+    l += Nn * std::log(2.0 * std::numbers::pi);
+    return 0.5 * l / Nn;
+}
+
+static void gradient_results(const Model &m, const double *t, const double *sums, const int trainable[3], double *loss_out, double grad[3])
+{
+    const double Nn = static_cast<double>(m.n);
+    *loss_out = loss_of(m, t);
+    grad[0] = trainable[0] ? 0.5 / Nn * (sums[0] - sums[2]) : 0.0;
+    grad[1] = trainable[1] ? 0.5 / Nn * (sums[1] - sums[3]) : 0.0;
+    grad[2] = trainable[2] ? sigmoid(to_unconstrained(m.sek.noise, true)) * (0.5 / Nn * (sums[4] - t[2])) : 0.0;
+}
+
 // Loss and softplus-space gradient at theta. K^-1 is formed as W^T W with
-// W = L^-1 (recursive TRSM on the triangular identity, then one triangular
-// MFMA product), n^3 flops in total instead of the reference's explicit
-// 2 n^3 double solve (core/src/cpu/gp_functions.cpp:953-966); the trace and
-// quadratic terms of core/src/cpu/tiled_algorithms.cpp:296-426 then come from
-// one fused pass over the lower triangle of K^-1.
+// W = L^-1, n^3 flops in total instead of the reference's explicit 2 n^3
+// double solve (core/src/cpu/gp_functions.cpp:953-966); the trace and quadratic
+// terms of core/src/cpu/tiled_algorithms.cpp:296-426 come from the lower
+// triangle of K^-1. Sizes that factor in one launch take W^T from identity
+// rows that ride along, and reduce each tile of K^-1 where it is formed
+// (measured on MI355X, with the blocked solve on the panel schedule's
+// factor / so: n = 1024 1.42 / 0.45 ms, 4096 6.5 / 2.8, 8192 20.0 / 13.9, 12288
+// 48.3 / 45.2); larger ones fit a model and use model_gradient().
 void loss_gradient(Context &c,
                    const double *x,
                    std::size_t x_len,
@@ -1677,8 +1698,43 @@ void loss_gradient(Context &c,
                    double grad[3])
 {
     Model m;
-    fit(c, m, x, x_len, y, y_len, n, r, theta, GPRAT_PRECISION_FP64);
-    model_gradient(m, trainable, loss_out, grad);
+    const int n_pad = static_cast<int>(padded(n));
+    if (!(trainable[0] || trainable[1] || trainable[2]) || !one_launch(n_pad, false))
+    {
+        fit(c, m, x, x_len, y, y_len, n, r, theta, GPRAT_PRECISION_FP64);
+        model_gradient(m, trainable, loss_out, grad);
+        return;
+    }
+    // identity rows ride along in the factorisation and leave as W^T = L^-T,
+    // a row of targets as z = L^-1 y; then alpha = W^T z
+    require(y != nullptr && y_len >= static_cast<std::size_t>(n), "training output must hold n values");
+    check_training(x, x_len, n, r, theta, GPRAT_PRECISION_FP64);
+    c.make_current();
+    const long lda = leading_dim(n_pad);
+    DevBuf<double> X(c, static_cast<std::size_t>(n_pad + 64) * lda);
+    double *z = X.get() + static_cast<long>(n_pad) * lda;
+    m.y = DevBuf<double>(c, n_pad);
+    k::fill(c.main, m.y.get(), n_pad, 0.0);
+    upload(c, m.y.get(), y, static_cast<std::size_t>(n));
+    GP_HIP(hipMemcpyAsync(z, m.y.get(), sizeof(double) * n_pad, hipMemcpyDeviceToDevice, c.main));
+    factor(c, m, x, x_len, n, r, theta, GPRAT_PRECISION_FP64, { X.get(), n_pad + 64, n_pad }, false);
+    m.alpha = DevBuf<double>(c, n_pad);
+    {
+        Timed t(c, c.main, "solve");
+        k::rowdot(c.main, X.get(), lda, n_pad, n_pad, z, m.alpha.get(), false, true);
+    }
+    k::loss_terms(c.main, m.L.get(), m.lda, m.y.get(), m.alpha.get(), m.n, c.scalars.get());
+    DevBuf<double> part(c, static_cast<std::size_t>(k::flow_gradient_tiles(n_pad)) * 5);
+    {
+        Timed t(c, c.main, "gradient");
+        k::flow_gradient(c.main, X.get(), lda, n_pad, m.x.get(), m.alpha.get(), r, m.sek, sigmoid(to_unconstrained(m.sek.lengthscale, false)),
+                         sigmoid(to_unconstrained(m.sek.vertical, false)), n, part.get(), c.scalars.get() + 8);
+    }
+    double h[13];
+    GP_HIP(hipMemcpyAsync(h, c.scalars.get(), sizeof h, hipMemcpyDefault, c.main));
+    c.sync();
+    check_pivots(c);
+    gradient_results(m, h, h + 8, trainable, loss_out, grad);
 }
 
 void model_gradient(Model &m, const int trainable[3], double *loss_out, double grad[3])
@@ -1690,12 +1746,7 @@ void model_gradient(Model &m, const int trainable[3], double *loss_out, double g
     double t[3];
     GP_HIP(hipMemcpyAsync(t, c.scalars.get(), sizeof t, hipMemcpyDefault, c.main));
     c.sync();
-    const double Nn = static_cast<double>(n);
-    {
-        double l = t[0] + t[1];
-        l += Nn * std::log(2.0 * std::numbers::pi);
-        *loss_out = 0.5 * l / Nn;
-    }
+    *loss_out = loss_of(m, t);
     grad[0] = grad[1] = grad[2] = 0.0;
     if (!(trainable[0] || trainable[1] || trainable[2]))
         return;
@@ -1731,7 +1782,6 @@ void model_gradient(Model &m, const int trainable[3], double *loss_out, double g
     W.reset();
     const double sig_l = sigmoid(to_unconstrained(m.sek.lengthscale, false));
     const double sig_v = sigmoid(to_unconstrained(m.sek.vertical, false));
-    const double sig_n = sigmoid(to_unconstrained(m.sek.noise, true));
     DevBuf<double> part(c, static_cast<std::size_t>(k::grad_tiles(n)) * 5);
     {
         Timed tm(c, c.main, "gradient");
@@ -1741,13 +1791,7 @@ void model_gradient(Model &m, const int trainable[3], double *loss_out, double g
     double sums[5];
     GP_HIP(hipMemcpyAsync(sums, c.scalars.get() + 8, sizeof sums, hipMemcpyDefault, c.main));
     c.sync();
-    // core/src/cpu/gp_optimizer.cpp:222-225 and tiled_algorithms.cpp:413-426
-    if (trainable[0])
-        grad[0] = 0.5 / Nn * (sums[0] - sums[2]);
-    if (trainable[1])
-        grad[1] = 0.5 / Nn * (sums[1] - sums[3]);
-    if (trainable[2])
-        grad[2] = sig_n * (0.5 / Nn * (sums[4] - t[2]));
+    gradient_results(m, t, sums, trainable, loss_out, grad);
 }
 
 void cholesky_tiles(Model &m, int T, int b, double *out)

@@ -268,10 +268,13 @@ void cholesky_fp64(Context &c, double *A, long lda, int n_pad, double *Winv);
 // extra: rows below the n_pad x n_pad matrix (A holds n_pad + extra rows)
 // that the factorisation treats as rows of L below it: on return they hold
 // B L^-T for the B they held (the forward solve of their transposes).
-// Their rows start at X (row stride lda; null: right below A). The factor is
+// Their rows start at X (row stride lda; null: right below A); the first
+// `unit` of them are identity rows that need not be stored (both
+// one_launch() sizes only). The factor is
 // complete in stream order on c.main; c.sync() and check_pivots() report a
 // pivot that was not positive.
-void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel = nullptr, int extra = 0, double *X = nullptr);
+void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel = nullptr, int extra = 0, double *X = nullptr,
+              int unit = 0);
 // After cholesky() and a c.sync(): throws GPRAT_ERR_NOT_SPD if a pivot was
 // not positive.
 void check_pivots(Context &c);
@@ -284,11 +287,16 @@ void solve_spd(Context &c, const double *L, long lda, const double *Winv, int n_
 void trsm_blocked(Context &c, const double *L, long lda, const double *Winv, const double *Wpanel, int wblock, int n_pad, double *B,
                   long ldb, int ncols, bool tri_rhs, double *out, long ldo);
 
-// rhs: a block row (64 x m.lda) that rides along and leaves as rhs L^-T
-// (one_launch() sizes only). keep_inverses: the panels' whole inverses, which
-// the solves step through, are wanted. Pivots as cholesky().
+// Rows that ride along in a factorisation (cholesky(), one_launch() sizes).
+struct Riding
+{
+    double *X = nullptr;
+    int extra = 0, unit = 0;
+};
+// keep_inverses: the panels' whole inverses, which the solves step through,
+// are wanted. Pivots as cholesky().
 void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int r, const double theta[3], int precision,
-            double *rhs = nullptr, bool keep_inverses = true);
+            Riding riding = {}, bool keep_inverses = true);
 void fit(Context &c,
          Model &m,
          const double *x,

@@ -436,6 +436,12 @@ void gradient_sums(hipStream_t s,
     hipLaunchKernelGGL(k_grad_partial, dim3(static_cast<unsigned>(tiles)), dim3(THREADS), 0, s, Kinv, lda, x, alpha, r, sek.scale(),
                        fl, sig_v, n, static_cast<int>(tiles), part);
     GP_CHECK_LAUNCH();
+    gradient_reduce(s, part, tiles, out);
+}
+
+void gradient_reduce(hipStream_t s, const double *part, long tiles, double *out)
+{
+    require(tiles >= 1 && tiles < (1L << 31), "gradient_reduce: bad shape");
     hipLaunchKernelGGL(k_grad_reduce, dim3(1), dim3(THREADS), 0, s, part, static_cast<int>(tiles), out);
     GP_CHECK_LAUNCH();
 }

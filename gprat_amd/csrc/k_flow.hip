@@ -50,7 +50,7 @@ struct FlowArgs
     double *A;
     long lda;
     double *X;
-    int nb, ne, unit;
+    int nb, ne, nu;
     double *Winv;
     int *info, *queue, *progress, *applied;
     int tasks;
@@ -368,6 +368,10 @@ __device__ __forceinline__ void diagonal_task(const FlowArgs &a, int q, double *
     }
 }
 
+// The unit row (its block column) at place `x` of a list of rows below the
+// matrix, or -1.
+__device__ __forceinline__ int extra_unit(const FlowArgs &a, int x) { return x < a.ne - a.nu ? -1 : x - (a.ne - a.nu); }
+
 // Tile (i, j) off the diagonal. unit >= 0: a row that starts from the identity
 // in block column `unit`.
 __device__ __forceinline__ void off_task(const FlowArgs &a, int i, int j, int unit, double *buf0, double *buf1, int *words, int &turn)
@@ -434,24 +438,26 @@ __device__ __forceinline__ void update_task(const FlowArgs &a, int i, int j, int
     publish(applied_of(a, i, j), p + 1);
 }
 
-// Rows below the matrix that panel p's updates of later columns reach.
-__host__ __device__ __forceinline__ int updated_extra(int ne, int unit, int p)
+// Rows below the matrix: nu that start from the identity (X's first nu), then
+// ne - nu others. A task list has the others first. Those that panel p's
+// updates of later columns reach:
+__host__ __device__ __forceinline__ int updated_extra(int ne, int nu, int p)
 {
     const int reach = (p + 1) * PANEL;
-    return unit && reach < ne ? reach : ne;
+    return (ne - nu) + (reach < nu ? reach : nu);
 }
 
 // Tasks of block column j: its tiles and its share of panel j / PANEL - 1's
 // updates [*u0, *u0 + *updates).
-__host__ __device__ __forceinline__ int column_tiles(int nb, int ne, int unit, int j) { return (nb - 1 - j) + (unit && j + 1 < ne ? j + 1 : ne); }
-__host__ __device__ __forceinline__ void column_updates(int nb, int ne, int unit, int j, long *u0, int *updates)
+__host__ __device__ __forceinline__ int column_tiles(int nb, int ne, int nu, int j) { return (nb - 1 - j) + (ne - nu) + (j + 1 < nu ? j + 1 : nu); }
+__host__ __device__ __forceinline__ void column_updates(int nb, int ne, int nu, int j, long *u0, int *updates)
 {
     const int p = j / PANEL - 1, m = nb - (p + 2) * PANEL;
     *u0 = 0;
     *updates = 0;
     if (p < 0 || m <= 0)
         return;
-    const long all = static_cast<long>(m) * (m + 1) / 2 + static_cast<long>(m) * updated_extra(ne, unit, p);
+    const long all = static_cast<long>(m) * (m + 1) / 2 + static_cast<long>(m) * updated_extra(ne, nu, p);
     const int c = j % PANEL;
     // rounded up: the first tile, which the next panel's first diagonal
     // block needs, is in the first share
@@ -469,7 +475,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) vo
     int turn = 0;
     int j = 0, first = 1;  // the current column and its first task's number
     long u0 = 0;
-    int updates = 0, tiles = column_tiles(a.nb, a.ne, a.unit, 0);
+    int updates = 0, tiles = column_tiles(a.nb, a.ne, a.nu, 0);
     for (;;)
     {
         __syncthreads();  // the previous task's LDS reads are done
@@ -489,8 +495,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) vo
         {
             first += tiles + updates;
             j++;
-            tiles = column_tiles(a.nb, a.ne, a.unit, j);
-            column_updates(a.nb, a.ne, a.unit, j, &u0, &updates);
+            tiles = column_tiles(a.nb, a.ne, a.nu, j);
+            column_updates(a.nb, a.ne, a.nu, j, &u0, &updates);
         }
         const int idx = t - first, below = a.nb - 1 - j;
         if (below > 0 && idx == 0)
@@ -498,18 +504,88 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) vo
         else if (idx < below)
             off_task(a, j + 1 + idx, j, -1, buf0, buf1, words, turn);
         else if (idx < tiles)
-            off_task(a, a.nb + idx - below, j, a.unit ? idx - below : -1, buf0, buf1, words, turn);
+        {
+            const int u = extra_unit(a, idx - below);
+            off_task(a, a.nb + (u >= 0 ? u : a.nu + idx - below), j, u, buf0, buf1, words, turn);
+        }
         else
         {
-            const int p = j / PANEL - 1, extra = updated_extra(a.ne, a.unit, p);
+            const int p = j / PANEL - 1, extra = updated_extra(a.ne, a.nu, p);
             long u = u0 + (idx - tiles);
             int c = (p + 2) * PANEL;
             while (u >= (a.nb - c) + extra)
                 u -= (a.nb - c++) + extra;
             const int r = static_cast<int>(u), own = a.nb - c;
-            update_task(a, r < own ? c + r : a.nb + r - own, c, p, a.unit && r >= own ? r - own : -1, buf0, buf1, words, turn);
+            const int e = r < own ? -1 : extra_unit(a, r - own);
+            update_task(a, r < own ? c + r : a.nb + (e >= 0 ? e : a.nu + r - own), c, p, e, buf0, buf1, words, turn);
         }
     }
+}
+
+// One 64x64 tile of K^-1 = WT WT^T per workgroup (i >= j; the sum starts at
+// block i, where row i of WT does; tiles in row order, so the longest sums
+// first), then k_grad_partial's sums over it.
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_flow_gradient(const double *WT, long ldw, int nb, const double *__restrict__ x,
+                                                                                                   const double *__restrict__ alpha, int r, double scale,
+                                                                                                   double fl, double sv, int n, double *__restrict__ part)
+{
+    __shared__ alignas(16) double buf0[NB * blk::XS];
+    __shared__ alignas(16) double buf1[NB * blk::XS];
+    const int tid = threadIdx.x;
+    const long t = blockIdx.x;
+    int ti = static_cast<int>((sqrt(8.0 * static_cast<double>(t) + 1.0) - 1.0) / 2.0);
+    while (static_cast<long>(ti) * (ti + 1) / 2 > t)
+        ti--;
+    while (static_cast<long>(ti + 1) * (ti + 2) / 2 <= t)
+        ti++;
+    const int tj = static_cast<int>(t - static_cast<long>(ti) * (ti + 1) / 2);
+    blk::v4d acc[2][2];
+    blk::zero(acc);
+    stream_blocks(WT + static_cast<long>(NB) * ti * ldw, WT + static_cast<long>(NB) * tj * ldw, ldw, ti, nb, buf0, buf1, tid,
+                  [&] { blk::mfma_nt_acc(buf0, buf1, acc); });
+    __syncthreads();
+    blk::for_each(acc, [&](int rr, int c, double v) { buf0[rr * blk::XS + c] = v; });
+    __syncthreads();
+    const int c = tid % NB;
+    const long j = static_cast<long>(tj) * NB + c;
+    double s[5] = { 0.0, 0.0, 0.0, 0.0, 0.0 };
+    if (j < n)
+    {
+        const double aj = alpha[j];
+        for (int rr = tid / NB; rr < NB; rr += THREADS / NB)
+        {
+            const long i = static_cast<long>(ti) * NB + rr;
+            if (i >= n || i < j)
+                continue;
+            const double kij = buf0[rr * blk::XS + c];
+            const double D = scale * window_sqdist(x, i, x, j, r);
+            const double e = exp(D);
+            const double dkl = fl * D * e;
+            const double dkv = e * sv;
+            const double w = (i == j) ? 1.0 : 2.0;
+            const double aa = alpha[i] * aj;
+            s[0] += w * kij * dkl;
+            s[1] += w * kij * dkv;
+            s[2] += w * aa * dkl;
+            s[3] += w * aa * dkv;
+            if (i == j)
+                s[4] += kij;
+        }
+    }
+    double(*red)[THREADS] = reinterpret_cast<double(*)[THREADS]>(buf1);
+#pragma unroll
+    for (int q = 0; q < 5; q++)
+        red[q][tid] = s[q];
+    __syncthreads();
+    for (int w = THREADS / 2; w > 0; w >>= 1)
+    {
+        if (tid < w)
+            for (int q = 0; q < 5; q++)
+                red[q][tid] += red[q][tid + w];
+        __syncthreads();
+    }
+    if (tid < 5)
+        part[t * 5 + tid] = red[tid][0];
 }
 
 }  // namespace
@@ -519,7 +595,7 @@ long flow_counters(int nb, int ne) { return 1 + (static_cast<long>(nb) + ne) * (
 void flow_cholesky(hipStream_t s, const FlowCall &f, int cus)
 {
     require(f.nb >= 1 && f.ne >= 0 && f.lda % 2 == 0 && f.lda >= static_cast<long>(NB) * f.nb, "flow_cholesky: bad shape");
-    require(!f.unit || f.ne <= f.nb, "flow_cholesky: more unit rows than columns");
+    require(f.nu >= 0 && f.nu <= f.ne && f.nu <= f.nb, "flow_cholesky: more unit rows than columns");
     require(f.ne == 0 || (f.X != nullptr && reinterpret_cast<uintptr_t>(f.X) % 16 == 0), "flow_cholesky: bad rows below the matrix");
     require(reinterpret_cast<uintptr_t>(f.A) % 16 == 0 && reinterpret_cast<uintptr_t>(f.Winv) % 16 == 0,
             "flow_cholesky: operands must be 16-byte aligned");
@@ -528,19 +604,34 @@ void flow_cholesky(hipStream_t s, const FlowCall &f, int cus)
     {
         long u0;
         int updates;
-        column_updates(f.nb, f.ne, f.unit, j, &u0, &updates);
-        tasks += column_tiles(f.nb, f.ne, f.unit, j) + updates;
+        column_updates(f.nb, f.ne, f.nu, j, &u0, &updates);
+        tasks += column_tiles(f.nb, f.ne, f.nu, j) + updates;
     }
     // every running workgroup may add one number past the last task
     require(tasks < (1L << 30), "flow_cholesky: too many tiles");
     const long counters = flow_counters(f.nb, f.ne);
-    const FlowArgs a{ f.A, f.lda, f.X, f.nb, f.ne, f.unit ? 1 : 0, f.Winv, f.info, f.counters, f.counters + 1, f.counters + 1 + f.nb + f.ne,
+    const FlowArgs a{ f.A, f.lda, f.X, f.nb, f.ne, f.nu, f.Winv, f.info, f.counters, f.counters + 1, f.counters + 1 + f.nb + f.ne,
                       static_cast<int>(tasks) };
     hipLaunchKernelGGL(k_flow_init, dim3(static_cast<unsigned>(ceil_div(counters, THREADS))), dim3(THREADS), 0, s, a, counters);
     GP_CHECK_LAUNCH();
     const long wgs = std::min<long>(tasks, 2L * cus);  // two workgroups' LDS fit a CU
     hipLaunchKernelGGL(k_flow, dim3(static_cast<unsigned>(wgs)), dim3(THREADS), 0, s, a);
     GP_CHECK_LAUNCH();
+}
+
+long flow_gradient_tiles(int n_pad) { return static_cast<long>(n_pad / NB) * (n_pad / NB + 1) / 2; }
+
+void flow_gradient(hipStream_t s, const double *WT, long ldw, int n_pad, const double *x, const double *alpha, int r, SEK sek, double sig_l,
+                   double sig_v, int n, double *part, double *out)
+{
+    const long tiles = flow_gradient_tiles(n_pad);
+    require(n >= 1 && n <= n_pad && n_pad % NB == 0 && ldw % 2 == 0 && ldw >= n_pad && tiles < (1L << 31), "flow_gradient: bad shape");
+    require(reinterpret_cast<uintptr_t>(WT) % 16 == 0, "flow_gradient: operand must be 16-byte aligned");
+    const double fl = -2.0 * sek.vertical / sek.lengthscale * sig_l;
+    hipLaunchKernelGGL(k_flow_gradient, dim3(static_cast<unsigned>(tiles)), dim3(THREADS), 0, s, WT, ldw, n_pad / NB, x, alpha, r, sek.scale(), fl,
+                       sig_v, n, part);
+    GP_CHECK_LAUNCH();
+    gradient_reduce(s, part, tiles, out);
 }
 
 }  // namespace gpamd::k

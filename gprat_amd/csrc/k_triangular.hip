@@ -558,7 +558,7 @@ __global__ __launch_bounds__(64 * COLDOT_WAVES) void k_coldot(const double *__re
 }
 
 // out[i] = (or -=) sum_{c < K} M[i * ld + c] v[c] for i < N, K a multiple
-// of 64. Each wavefront owns four consecutive rows: lane l reads columns
+// of 64 (upper: from the columns of row i's 64x64 diagonal block on). Each wavefront owns four consecutive rows: lane l reads columns
 // l, l + 64, ... of each (coalesced 512-byte segments), then every row sum
 // is reduced across the wavefront by a fixed butterfly.
 __global__ __launch_bounds__(THREADS) void k_rowdot(const double *__restrict__ M,
@@ -567,7 +567,8 @@ __global__ __launch_bounds__(THREADS) void k_rowdot(const double *__restrict__ M
                                                      int N,
                                                      const double *__restrict__ v,
                                                      double *__restrict__ out,
-                                                     bool sub)
+                                                     bool sub,
+                                                     bool upper)
 {
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -576,7 +577,7 @@ __global__ __launch_bounds__(THREADS) void k_rowdot(const double *__restrict__ M
         return;
     const int rows = min(4, N - i0);
     double s[4] = { 0.0, 0.0, 0.0, 0.0 };
-    for (int c0 = 0; c0 < K; c0 += 256)
+    for (int c0 = upper ? i0 / NB * NB : 0; c0 < K; c0 += 256)
     {
         double m[4][4], x[4];
 #pragma unroll
@@ -986,10 +987,10 @@ void coldot(hipStream_t s, const double *M, long ld, int K, int N, const double 
     GP_CHECK_LAUNCH();
 }
 
-void rowdot(hipStream_t s, const double *M, long ld, int K, int N, const double *v, double *out, bool sub)
+void rowdot(hipStream_t s, const double *M, long ld, int K, int N, const double *v, double *out, bool sub, bool upper)
 {
     require(K >= 64 && K % 64 == 0 && N >= 1 && ld >= K, "rowdot: bad shape");
-    hipLaunchKernelGGL(k_rowdot, dim3(ceil_div(N, 16)), dim3(THREADS), 0, s, M, ld, K, N, v, out, sub);
+    hipLaunchKernelGGL(k_rowdot, dim3(ceil_div(N, 16)), dim3(THREADS), 0, s, M, ld, K, N, v, out, sub, upper);
     GP_CHECK_LAUNCH();
 }
 

@@ -89,6 +89,8 @@ void gradient_sums(hipStream_t s,
                    int n,
                    double *part,
                    double *out);
+// out[q] = sum of part[5 t + q] over t < tiles (fixed order).
+void gradient_reduce(hipStream_t s, const double *part, long tiles, double *out);
 
 // ---- dense products on MFMA (k_gemm.hip) ----------------------------------
 
@@ -299,7 +301,7 @@ constexpr int FLOW_PANEL = 8;
 // A: the lower triangle of an nb x nb matrix of 64x64 blocks (row stride
 // lda), factored in place. X: ne block rows of the same width and stride that
 // leave as X L^-T (rows are independent, so what unused ones hold does not
-// matter). unit: those rows start as the identity's first ne block rows
+// matter); the first nu of them start as the identity's first nu block rows
 // instead (X is not read; the blocks left of a row's first nonzero one are not
 // written). The row-major inverses of L's 64x64 diagonal blocks
 // go to Winv. counters: flow_counters(nb, ne) ints; info: the smallest
@@ -310,13 +312,20 @@ struct FlowCall
     double *A;
     long lda;
     double *X;
-    int nb, ne;
-    bool unit;
+    int nb, ne, nu;
     double *Winv;
     int *info, *counters;
 };
 long flow_counters(int nb, int ne);
 void flow_cholesky(hipStream_t s, const FlowCall &f, int cus);
+
+// The sums of gradient_sums() (k_covariance.hip) straight from WT = L^-T
+// (n_pad x n_pad, row stride ldw, not read left of a row's diagonal block):
+// each 64x64 tile of K^-1 = WT WT^T on or below the diagonal is formed in
+// registers and reduced there. part: flow_gradient_tiles(n_pad) * 5 doubles.
+long flow_gradient_tiles(int n_pad);
+void flow_gradient(hipStream_t s, const double *WT, long ldw, int n_pad, const double *x, const double *alpha, int r, SEK sek, double sig_l,
+                   double sig_v, int n, double *part, double *out);
 
 // Block steps of the vector solves with the saved diagonal-block inverses
 // Winv (block J at Winv + J*64*64). Forward: out[J] = W_JJ rhs[J],
@@ -331,7 +340,8 @@ void solve_upper_step(hipStream_t s, const double *L, long lda, const double *Wi
 // rowdot: out[i] = (or -=) sum_{c<K} M[i][c] v[c], i < N, K % 64 == 0.
 // v must not overlap out.
 void coldot(hipStream_t s, const double *M, long ld, int K, int N, const double *v, double *out, bool sub);
-void rowdot(hipStream_t s, const double *M, long ld, int K, int N, const double *v, double *out, bool sub);
+// rowdot with upper: M is zero, and not read, left of each row's 64x64 diagonal block.
+void rowdot(hipStream_t s, const double *M, long ld, int K, int N, const double *v, double *out, bool sub, bool upper = false);
 
 // Inverses of the 256-wide diagonal blocks of L covering rows
 // [row0, row0 + rows) (the last block may be narrower), built from the
