@@ -490,13 +490,24 @@ static void flow(Context &c, double *A, long lda, int n_pad, double *Winv, doubl
     Timed t(c, c.main, "cholesky");
     const int nb = n_pad / 64, ne = extra / 64;
     DevBuf<int> counters(c, static_cast<std::size_t>(k::flow_counters(nb, ne)));
-    k::flow_cholesky(c.main, k::FlowCall{ A, lda, X, nb, ne, unit / 64, Winv, c.info.get(), counters.get() }, c.cus);
+    k::flow_cholesky(c.main, k::FlowCall{ A, lda, X, nb, ne, unit / 64, false, Winv, c.info.get(), counters.get() }, c.cus);
     if (Wpanel)
     {
         const int width = outer_block(n_pad);
         DevBuf<double> tmp(c, static_cast<std::size_t>(std::max(1L, k::panel_inverses_scratch(n_pad, width))));
         k::panel_inverses(c.main, A, lda, Winv, n_pad, width, Wpanel, tmp.get());
     }
+    GP_HIP(hipMemcpyAsync(c.host_info, c.info.get(), sizeof(int), hipMemcpyDeviceToHost, c.main));
+}
+
+// X L^-T in place for `rows` rows X (row stride lda, as L; the first `unit`
+// of them identity rows, see cholesky()) by the same launch on a given factor.
+static void flow_solve(Context &c, const double *L, long lda, int n_pad, const double *Winv, double *X, int rows, int unit = 0)
+{
+    const int nb = n_pad / 64, ne = rows / 64;
+    DevBuf<int> counters(c, static_cast<std::size_t>(k::flow_counters(nb, ne)));
+    k::flow_cholesky(c.main, k::FlowCall{ const_cast<double *>(L), lda, X, nb, ne, unit / 64, true, const_cast<double *>(Winv), c.info.get(), counters.get() },
+                     c.cus);
     GP_HIP(hipMemcpyAsync(c.host_info, c.info.get(), sizeof(int), hipMemcpyDeviceToHost, c.main));
 }
 
@@ -1163,6 +1174,7 @@ void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int
     m.lda = leading_dim(m.n_pad);
     m.sek = SEK{ theta[0], theta[1], theta[2] };
     m.precision = precision;
+    m.fp32_updates = precision == GPRAT_PRECISION_MIXED && !one_launch(m.n_pad, true);
     const std::size_t xl = static_cast<std::size_t>(n) + r - 1;
     m.x = DevBuf<double>(c, xl);
     m.L = DevBuf<double>(c, static_cast<std::size_t>(m.n_pad) * m.lda);
@@ -1177,7 +1189,7 @@ void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int
     }
     cholesky(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), precision == GPRAT_PRECISION_MIXED, m.Wpanel.get(),
              riding.extra, riding.X, riding.unit);
-    if (precision == GPRAT_PRECISION_MIXED)
+    if (m.fp32_updates)
     {
         // the covariance's strictly lower part, for the FP64 residual of the
         // variance refinement, goes to the factor's free upper triangle
@@ -1284,6 +1296,110 @@ void fit(Context &c,
     }
 }
 
+// Work on the second stream beside c.main: it starts after what c.main holds,
+// and c.main waits for it at join(), at the latest when this goes out of scope
+// (an exception included), so buffers declared before it outlive it in
+// stream order. Off (or with one stream) the work is c.main's own.
+class SideStream
+{
+  public:
+    SideStream(Context &c, bool on) : c_(c), on_(on && c.panel != c.main)
+    {
+        if (!on_)
+            return;
+        hipEvent_t e = c_.event();
+        const hipError_t r = hipEventRecord(e, c_.main);
+        const hipError_t w = r == hipSuccess ? hipStreamWaitEvent(c_.panel, e, 0) : r;
+        c_.recycle(e);
+        GP_HIP(w);
+    }
+    SideStream(const SideStream &) = delete;
+    SideStream &operator=(const SideStream &) = delete;
+    ~SideStream()
+    {
+        if (!on_)
+            return;
+        done_ = done_ ? done_ : c_.event();
+        (void)hipEventRecord(done_, c_.panel);
+        (void)hipStreamWaitEvent(c_.main, done_, 0);
+        c_.recycle(done_);
+    }
+    hipStream_t stream() const { return on_ ? c_.panel : c_.main; }
+    void done()
+    {
+        if (on_ && !done_)
+        {
+            done_ = c_.event();
+            GP_HIP(hipEventRecord(done_, c_.panel));
+        }
+    }
+    void join()
+    {
+        done();
+        if (on_)
+        {
+            GP_HIP(hipStreamWaitEvent(c_.main, done_, 0));
+            c_.recycle(done_);
+            on_ = false;
+        }
+    }
+
+  private:
+    Context &c_;
+    bool on_;
+    hipEvent_t done_ = nullptr;
+};
+
+// How the forward solves of mt test points run, by the size of V = L^-1 K*^T.
+// Measured on MI355X (predictions with variance, blocked solve / one launch /
+// few rows, ms; m test points):
+//   n = 1024  m = 1 0.37 / 0.20 / 0.11, m = 1024 0.37 / 0.27 / 0.19, m = 4096 0.39 / 0.44 / 0.34
+//   n = 4096  m = 100 1.27 / 0.58 / 0.36, m = 1024 1.33 / 0.91 / 0.88, m = 2048 1.57 / 1.27 / 1.55
+//   n = 8192  m = 16 2.25 / 1.10 / 0.33, m = 512 2.21 / 1.62 / 1.48, m = 2048 3.58 / 4.03 / -
+//   n = 16384 m = 256 4.18 / 3.23 / 2.90, m = 700 6.36 / 5.83 / 6.91
+//   n = 32768 m = 128 9.65 / 6.56 / 5.99, m = 256 11.6 / 9.46 / 10.5
+// The few-row kernels read L once per 64 rows with no stage between memory and
+// the matrix cores; the one launch reuses tiles through LDS but pays a
+// hand-over per 64 columns; the blocked solve's 128x128 tiles need large
+// products.
+enum class ForwardSolve
+{
+    FewRows,
+    OneLaunch,
+    Blocked
+};
+static ForwardSolve forward_solve(const FactorView &m, int mt)
+{
+    const long size = static_cast<long>(m.n_pad) * round_up(mt, 64);
+    if (const char *e = std::getenv("GPRAT_FORWARD_SOLVE"))
+        return std::atoi(e) == 0 && m.Wpanel ? ForwardSolve::FewRows : (std::atoi(e) <= 1 ? ForwardSolve::OneLaunch : ForwardSolve::Blocked);
+    if (m.Wpanel && size <= 4L << 20)
+        return ForwardSolve::FewRows;
+    return size <= 10L << 20 ? ForwardSolve::OneLaunch : ForwardSolve::Blocked;
+}
+
+// K* L^-T (the rows of V^T) for mt test points by one of the row methods:
+// rows of m.lda values, zero past mt and n (mt rounded up to 64 rows).
+static DevBuf<double> solved_rows(const FactorView &m, ForwardSolve how, const double *dz, int mt)
+{
+    Context &c = *m.ctx;
+    const int rows = static_cast<int>(round_up(mt, 64));
+    DevBuf<double> X(c, static_cast<std::size_t>(rows) * m.lda);
+    {
+        Timed t(c, c.main, "assemble");
+        k::assemble_cross_rows(c.main, m.x, dz, m.r, m.sek, X.get(), m.lda, m.n, m.n_pad, mt, rows);
+    }
+    Timed t(c, c.main, "trsm");
+    if (how == ForwardSolve::OneLaunch)
+    {
+        flow_solve(c, m.L, m.lda, m.n_pad, m.Winv, X.get(), rows);
+        return X;
+    }
+    DevBuf<double> V(c, static_cast<std::size_t>(rows) * m.lda);
+    k::few_rows_solve(c.main, m.L, m.lda, m.Wpanel, m.wblock, m.n_pad, X.get(), V.get(), m.lda, static_cast<int>(mt <= 32 ? round_up(mt, 16) : rows));
+    return V;
+}
+
 void predict_view(const FactorView &m, const double *z, std::size_t z_len, int mt, double *mean, double *var)
 {
     Context &c = *m.ctx;
@@ -1300,11 +1416,17 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
     const int splits = k::mean_splits(m.n, mt);
     DevBuf<double> partial(c, static_cast<std::size_t>(splits) * mt);
     DevBuf<double> dmean(c, mt);
+    const ForwardSolve how = m.mixed ? ForwardSolve::Blocked : forward_solve(m, mt);
+    // beside the row methods, whose launches leave most of the device idle,
+    // the mean's kernels run on the second stream
+    SideStream side(c, var && how != ForwardSolve::Blocked);
     {
-        Timed t(c, c.main, "mean");
-        k::predict_mean(c.main, m.x, dz.get(), m.alpha, m.r, m.sek, m.n, mt, partial.get(), splits, dmean.get());
+        Timed t(c, side.stream(), "mean");
+        k::predict_mean(side.stream(), m.x, dz.get(), m.alpha, m.r, m.sek, m.n, mt, partial.get(), splits, dmean.get());
     }
-    DevBuf<double> dvar;
+    side.done();
+    DevBuf<double> dvar, rows;
+    bool solved_here = false;  // by a dataflow launch: its completion is checked below
     if (var && m.mixed && m.refine_variance)
     {
         const int m_pad = static_cast<int>(round_up(mt, 64));
@@ -1321,6 +1443,16 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
         dvar = DevBuf<double>(c, mt);
         variance_colsq_f32(c, m, dz.get(), mt, m_pad, colsq.get());
         k::variance_finish(c.main, colsq.get(), m.sek.vertical, mt, dvar.get());
+        GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
+    }
+    else if (var && how != ForwardSolve::Blocked)
+    {
+        solved_here = how == ForwardSolve::OneLaunch;
+        DevBuf<double> sumsq(c, mt);
+        dvar = DevBuf<double>(c, mt);
+        rows = solved_rows(m, how, dz.get(), mt);
+        k::row_sumsq(c.main, rows.get(), m.lda, mt, m.n_pad, sumsq.get());
+        k::variance_finish(c.main, sumsq.get(), m.sek.vertical, mt, dvar.get());
         GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
     }
     else if (var)
@@ -1349,8 +1481,11 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
         k::variance_finish(c.main, colsq.get(), m.sek.vertical, mt, dvar.get());
         GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
     }
+    side.join();
     GP_HIP(hipMemcpyAsync(mean, dmean.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
     c.sync();
+    if (solved_here)
+        check_pivots(c);
 }
 
 // Mean and the whole latent posterior covariance Sigma = K** - V^T V,
@@ -1359,8 +1494,9 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
 // symmetric_matrix_matrix_tiled, tiled_algorithms.cpp:230-254) and returns
 // only its diagonal (gp_functions.cpp:663-695); here Sigma starts as K**
 // and every block V_J of the blocked solve subtracts V_J^T V_J on the
-// matrix cores, in step order. FP64 throughout (a mixed-precision model's
-// factor carries its own accuracy into Sigma).
+// matrix cores, in step order; the row methods keep V^T and subtract its rows'
+// products afterwards. FP64 throughout (a mixed-precision model's factor
+// carries its own accuracy into Sigma).
 void predict_full_cov_view(const FactorView &m, const double *z, std::size_t z_len, int mt, double *mean, double *cov)
 {
     Context &c = *m.ctx;
@@ -1374,6 +1510,22 @@ void predict_full_cov_view(const FactorView &m, const double *z, std::size_t z_l
     DevBuf<double> dz(c, zl);
     upload(c, dz.get(), z, zl);
     const int m_pad = static_cast<int>(round_up(mt, 64));
+    if (const ForwardSolve how = forward_solve(m, mt); how != ForwardSolve::Blocked)
+    {
+        DevBuf<double> S(c, static_cast<std::size_t>(m_pad) * m_pad);
+        k::assemble_cross_t(c.main, dz.get(), dz.get(), m.r, m.sek, S.get(), m_pad, mt, m_pad, mt, m_pad);
+        DevBuf<double> V = solved_rows(m, how, dz.get(), mt);
+        DevBuf<double> part(c, static_cast<std::size_t>(k::row_products_scratch(m.n_pad, m_pad)));
+        {
+            Timed t(c, c.main, "trsm");
+            k::subtract_row_products(c.main, V.get(), m.lda, m.n_pad, S.get(), m_pad, m_pad, part.get());
+        }
+        GP_HIP(hipMemcpy2DAsync(cov, sizeof(double) * mt, S.get(), sizeof(double) * m_pad, sizeof(double) * mt, mt, hipMemcpyDefault, c.main));
+        c.sync();
+        if (how == ForwardSolve::OneLaunch)
+            check_pivots(c);
+        return;
+    }
     DevBuf<double> B(c, static_cast<std::size_t>(m.n_pad) * m_pad), S(c, static_cast<std::size_t>(m_pad) * m_pad);
     {
         Timed t(c, c.main, "assemble");
@@ -1522,7 +1674,10 @@ FactorView view(const Model &m)
     FactorView v{ m.ctx, m.x.get(), m.n, m.n_pad, m.r, m.lda, m.sek, m.L.get(), m.Winv.get(), m.alpha.get(),
                   m.precision == GPRAT_PRECISION_MIXED, m.Wpanel.get(), m.wblock };
     v.refine_variance = m.refine_variance;
-    if (m.precision == GPRAT_PRECISION_MIXED)
+    // a factor without FP32 updates needs no refinement: its forward solve in
+    // FP64 is the refined variance
+    v.mixed = m.fp32_updates || (v.mixed && !m.refine_variance);
+    if (m.fp32_updates)
     {
         v.Kup = m.L.get();  // mixed models keep the covariance in the factor's strict upper triangle
         v.ldk = m.lda;
@@ -1750,6 +1905,26 @@ void model_gradient(Model &m, const int trainable[3], double *loss_out, double g
     grad[0] = grad[1] = grad[2] = 0.0;
     if (!(trainable[0] || trainable[1] || trainable[2]))
         return;
+    const double sig_l = sigmoid(to_unconstrained(m.sek.lengthscale, false));
+    const double sig_v = sigmoid(to_unconstrained(m.sek.vertical, false));
+    double sums[5];
+    if (one_launch(m.n_pad, false))
+    {
+        DevBuf<double> X(c, static_cast<std::size_t>(m.n_pad) * m.lda), part(c, static_cast<std::size_t>(k::flow_gradient_tiles(m.n_pad)) * 5);
+        {
+            Timed tm(c, c.main, "inverse");
+            flow_solve(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), X.get(), m.n_pad, m.n_pad);
+        }
+        {
+            Timed tm(c, c.main, "gradient");
+            k::flow_gradient(c.main, X.get(), m.lda, m.n_pad, m.x.get(), m.alpha.get(), r, m.sek, sig_l, sig_v, n, part.get(), c.scalars.get() + 8);
+        }
+        GP_HIP(hipMemcpyAsync(sums, c.scalars.get() + 8, sizeof sums, hipMemcpyDefault, c.main));
+        c.sync();
+        check_pivots(c);
+        gradient_results(m, t, sums, trainable, loss_out, grad);
+        return;
+    }
     const std::size_t elems = static_cast<std::size_t>(m.n_pad) * m.lda;
     DevBuf<double> W(c, elems);
     DevBuf<double> Kinv(c, elems);
@@ -1780,15 +1955,12 @@ void model_gradient(Model &m, const int trainable[3], double *loss_out, double g
         k::gemm_f64(c.main, g);
     }
     W.reset();
-    const double sig_l = sigmoid(to_unconstrained(m.sek.lengthscale, false));
-    const double sig_v = sigmoid(to_unconstrained(m.sek.vertical, false));
     DevBuf<double> part(c, static_cast<std::size_t>(k::grad_tiles(n)) * 5);
     {
         Timed tm(c, c.main, "gradient");
         k::gradient_sums(c.main, Kinv.get(), m.lda, m.x.get(), m.alpha.get(), r, m.sek, sig_l, sig_v, n, part.get(),
                          c.scalars.get() + 8);
     }
-    double sums[5];
     GP_HIP(hipMemcpyAsync(sums, c.scalars.get() + 8, sizeof sums, hipMemcpyDefault, c.main));
     c.sync();
     gradient_results(m, t, sums, trainable, loss_out, grad);

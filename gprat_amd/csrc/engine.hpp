@@ -202,6 +202,7 @@ struct Model
     long lda = 0;
     SEK sek{};
     int precision = GPRAT_PRECISION_FP64;
+    bool fp32_updates = false;   // mixed precision: the factorisation's trailing updates ran in FP32
     int refine_iterations = 0;   // mixed precision: refinement steps taken for alpha
     double refine_last = 0.0;    // last max|delta| / max|alpha|
     // mixed precision: the latent variance is refined in FP64 (the strict

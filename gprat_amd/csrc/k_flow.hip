@@ -50,7 +50,7 @@ struct FlowArgs
     double *A;
     long lda;
     double *X;
-    int nb, ne, nu;
+    int nb, ne, nu, solve;
     double *Winv;
     int *info, *queue, *progress, *applied;
     int tasks;
@@ -69,8 +69,9 @@ __global__ __launch_bounds__(THREADS) void k_flow_init(FlowArgs a, long counters
     const long i = static_cast<long>(blockIdx.x) * THREADS + threadIdx.x;
     if (i == 0)
         *a.info = INT_MAX;
+    // the queue, progress and applied counters lie one after another
     if (i < counters)
-        a.queue[i] = 0;  // the queue, progress and applied counters lie one after another
+        a.queue[i] = a.solve && i >= 1 && i <= a.nb ? a.nb : 0;
 }
 
 __device__ __forceinline__ int load_counter(const int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
@@ -306,6 +307,13 @@ __device__ __forceinline__ void diagonal_task(const FlowArgs &a, int q, double *
         blk::v4d off[2][2], dia[2][2];
         blk::zero(off);
         blk::zero(dia);
+        double *lqj = rq + static_cast<long>(NB) * j;
+        // the stored values first: their latency is then not the chain's
+        if (q / PANEL >= 2)
+            wait_for(a, applied_of(a, q, q), applied_of(a, q, q), q / PANEL - 1, applied_of(a, q, j), j / PANEL - 1, words, turn);
+        double s[16];
+        blk::load_at_acc(lqj, a.lda, s, tid);
+        blk::load_at_acc(dst, a.lda, d, tid);
         const int pair = first_product(q);  // both tiles' products from here on
         for (int k = first_product(j); k < j;)
         {
@@ -316,12 +324,6 @@ __device__ __forceinline__ void diagonal_task(const FlowArgs &a, int q, double *
                 stream_blocks(rq, rj, a.lda, k, k1, buf0, buf1, tid, [&] { mfma_pair(buf0, buf1, off, dia, tid); });
             k = k1;
         }
-        double *lqj = rq + static_cast<long>(NB) * j;
-        if (q / PANEL >= 2)
-            wait_for(a, applied_of(a, q, q), applied_of(a, q, q), q / PANEL - 1, applied_of(a, q, j), j / PANEL - 1, words, turn);
-        double s[16];
-        blk::load_at_acc(lqj, a.lda, s, tid);
-        blk::load_at_acc(dst, a.lda, d, tid);
         __syncthreads();
         stage_difference(buf0, s, off, tid);
         int e = 0;
@@ -373,7 +375,8 @@ __device__ __forceinline__ void diagonal_task(const FlowArgs &a, int q, double *
 __device__ __forceinline__ int extra_unit(const FlowArgs &a, int x) { return x < a.ne - a.nu ? -1 : x - (a.ne - a.nu); }
 
 // Tile (i, j) off the diagonal. unit >= 0: a row that starts from the identity
-// in block column `unit`.
+// in block column `unit`. SOLVE: the factor is given.
+template <bool SOLVE>
 __device__ __forceinline__ void off_task(const FlowArgs &a, int i, int j, int unit, double *buf0, double *buf1, int *words, int &turn)
 {
     const int tid = own_thread();
@@ -384,12 +387,8 @@ __device__ __forceinline__ void off_task(const FlowArgs &a, int i, int j, int un
     blk::zero(acc);
     const int before = j / PANEL - 1;                     // panels subtracted by update tasks
     const bool stored = unit < 0 || unit / PANEL < before;  // the tile has a stored value
-    for (int k = max(first_product(j), unit); k < j;)
-    {
-        const int k1 = min(j, wait_for(a, a.progress + i, a.progress + j, k + 1, words, turn));
-        stream_blocks(ri, rj, a.lda, k, k1, buf0, buf1, tid, [&] { blk::mfma_nt_acc(buf0, buf1, acc, tid); });
-        k = k1;
-    }
+    // the stored value, and a given factor's inverse block, first: their
+    // latency is then not the chain's
     double s[16];
     if (stored)
     {
@@ -402,10 +401,25 @@ __device__ __forceinline__ void off_task(const FlowArgs &a, int i, int j, int un
         int e = 0;
         blk::for_each(acc, [&](int r, int c, double) { s[e++] = (j == unit && r == c) ? 1.0 : 0.0; }, tid);
     }
+    const double *wj = a.Winv + static_cast<long>(j) * NB * NB;
+    blk::d2 vw[8];
+    if (SOLVE)
+        blk::load_block(wj, NB, vw, tid);
+    for (int k = max(first_product(j), unit); k < j;)
+    {
+        const int k1 = min(j, wait_for(a, a.progress + i, a.progress + j, k + 1, words, turn));
+        stream_blocks(ri, rj, a.lda, k, k1, buf0, buf1, tid, [&] { blk::mfma_nt_acc(buf0, buf1, acc, tid); });
+        k = k1;
+    }
     __syncthreads();
     stage_difference(buf0, s, acc, tid);
-    wait_for(a, a.progress + j, a.progress + j, j + 1, words, turn);
-    blk::stage_block(buf1, a.Winv + static_cast<long>(j) * NB * NB, NB, tid);
+    if (SOLVE)
+        blk::store_block(buf1, vw, tid);
+    else
+    {
+        wait_for(a, a.progress + j, a.progress + j, j + 1, words, turn);
+        blk::stage_block(buf1, wj, NB, tid);
+    }
     __syncthreads();
     blk::v4d l[4];
     solve_product(buf0, buf1, l, tid);
@@ -448,16 +462,21 @@ __host__ __device__ __forceinline__ int updated_extra(int ne, int nu, int p)
 }
 
 // Tasks of block column j: its tiles and its share of panel j / PANEL - 1's
-// updates [*u0, *u0 + *updates).
-__host__ __device__ __forceinline__ int column_tiles(int nb, int ne, int nu, int j) { return (nb - 1 - j) + (ne - nu) + (j + 1 < nu ? j + 1 : nu); }
-__host__ __device__ __forceinline__ void column_updates(int nb, int ne, int nu, int j, long *u0, int *updates)
+// updates [*u0, *u0 + *updates). Column c has own_tiles of the matrix's rows
+// from block `from` on (none when L is given).
+__host__ __device__ __forceinline__ int own_tiles(const FlowArgs &a, int from) { return a.solve ? 0 : a.nb - from; }
+__host__ __device__ __forceinline__ int column_tiles(const FlowArgs &a, int j)
 {
-    const int p = j / PANEL - 1, m = nb - (p + 2) * PANEL;
+    return own_tiles(a, j + 1) + (a.ne - a.nu) + (j + 1 < a.nu ? j + 1 : a.nu);
+}
+__host__ __device__ __forceinline__ void column_updates(const FlowArgs &a, int j, long *u0, int *updates)
+{
+    const int p = j / PANEL - 1, m = a.nb - (p + 2) * PANEL;
     *u0 = 0;
     *updates = 0;
     if (p < 0 || m <= 0)
         return;
-    const long all = static_cast<long>(m) * (m + 1) / 2 + static_cast<long>(m) * updated_extra(ne, nu, p);
+    const long all = (a.solve ? 0 : static_cast<long>(m) * (m + 1) / 2) + static_cast<long>(m) * updated_extra(a.ne, a.nu, p);
     const int c = j % PANEL;
     // rounded up: the first tile, which the next panel's first diagonal
     // block needs, is in the first share
@@ -466,6 +485,8 @@ __host__ __device__ __forceinline__ void column_updates(int nb, int ne, int nu, 
     *updates = static_cast<int>(hi - lo);
 }
 
+// SOLVE: the rows below a given factor only (a.solve).
+template <bool SOLVE>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_flow(FlowArgs a)
 {
     __shared__ alignas(16) double buf0[NB * blk::XS];
@@ -473,9 +494,9 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) vo
     __shared__ int words[2];
     __shared__ int next;
     int turn = 0;
-    int j = 0, first = 1;  // the current column and its first task's number
+    int j = 0, first = a.solve ? 0 : 1;  // the current column and its first task's number
     long u0 = 0;
-    int updates = 0, tiles = column_tiles(a.nb, a.ne, a.nu, 0);
+    int updates = 0, tiles = column_tiles(a, 0);
     for (;;)
     {
         __syncthreads();  // the previous task's LDS reads are done
@@ -485,37 +506,41 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) vo
         const int t = __builtin_amdgcn_readfirstlane(next);
         if (t >= a.tasks)
             return;
-        if (t == 0)
-        {
-            diagonal_task(a, 0, buf0, buf1, words, turn);
-            continue;
-        }
+        if constexpr (!SOLVE)
+            if (t == 0)
+            {
+                diagonal_task(a, 0, buf0, buf1, words, turn);
+                continue;
+            }
         // task numbers only grow: the walk is incremental
         while (t >= first + tiles + updates)
         {
             first += tiles + updates;
             j++;
-            tiles = column_tiles(a.nb, a.ne, a.nu, j);
-            column_updates(a.nb, a.ne, a.nu, j, &u0, &updates);
+            tiles = column_tiles(a, j);
+            column_updates(a, j, &u0, &updates);
         }
-        const int idx = t - first, below = a.nb - 1 - j;
-        if (below > 0 && idx == 0)
-            diagonal_task(a, j + 1, buf0, buf1, words, turn);
-        else if (idx < below)
-            off_task(a, j + 1 + idx, j, -1, buf0, buf1, words, turn);
+        const int idx = t - first, below = own_tiles(a, j + 1);
+        if (!SOLVE && idx < below)
+        {
+            if (idx == 0)
+                diagonal_task(a, j + 1, buf0, buf1, words, turn);
+            else
+                off_task<SOLVE>(a, j + 1 + idx, j, -1, buf0, buf1, words, turn);
+        }
         else if (idx < tiles)
         {
             const int u = extra_unit(a, idx - below);
-            off_task(a, a.nb + (u >= 0 ? u : a.nu + idx - below), j, u, buf0, buf1, words, turn);
+            off_task<SOLVE>(a, a.nb + (u >= 0 ? u : a.nu + idx - below), j, u, buf0, buf1, words, turn);
         }
         else
         {
             const int p = j / PANEL - 1, extra = updated_extra(a.ne, a.nu, p);
             long u = u0 + (idx - tiles);
             int c = (p + 2) * PANEL;
-            while (u >= (a.nb - c) + extra)
-                u -= (a.nb - c++) + extra;
-            const int r = static_cast<int>(u), own = a.nb - c;
+            while (u >= own_tiles(a, c) + extra)
+                u -= own_tiles(a, c++) + extra;
+            const int r = static_cast<int>(u), own = own_tiles(a, c);
             const int e = r < own ? -1 : extra_unit(a, r - own);
             update_task(a, r < own ? c + r : a.nb + (e >= 0 ? e : a.nu + r - own), c, p, e, buf0, buf1, words, turn);
         }
@@ -588,6 +613,56 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) vo
         part[t * 5 + tid] = red[tid][0];
 }
 
+// Partial sums of a 64x64 tile (i, j), i >= j, of V V^T over one of gridDim.y
+// shares of V's 64-blocks, then their fixed-order sum subtracted from both
+// halves of S. The tiles alone would leave most of the device idle (36 for
+// 512 rows), so the shares are cut to about one workgroup slot each.
+__device__ __forceinline__ void triangle_tile(int t, int &i, int &j)
+{
+    i = static_cast<int>((sqrt(8.0 * static_cast<double>(t) + 1.0) - 1.0) / 2.0);
+    while (i * (i + 1) / 2 > t)
+        i--;
+    while ((i + 1) * (i + 2) / 2 <= t)
+        i++;
+    j = t - i * (i + 1) / 2;
+}
+
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2))) void k_row_products(const double *V, long ldv, int nb, double *__restrict__ part)
+{
+    __shared__ alignas(16) double buf0[NB * blk::XS];
+    __shared__ alignas(16) double buf1[NB * blk::XS];
+    const int tid = threadIdx.x;
+    int i, j;
+    triangle_tile(blockIdx.x, i, j);
+    const int per = (nb + gridDim.y - 1) / gridDim.y;
+    const int k0 = min(nb, static_cast<int>(blockIdx.y) * per), k1 = min(nb, k0 + per);
+    blk::v4d acc[2][2];
+    blk::zero(acc);
+    if (k0 < k1)
+        stream_blocks(V + static_cast<long>(NB) * i * ldv, V + static_cast<long>(NB) * j * ldv, ldv, k0, k1, buf0, buf1, tid,
+                      [&] { blk::mfma_nt_acc(buf0, buf1, acc); });
+    double *p = part + (static_cast<long>(blockIdx.x) * gridDim.y + blockIdx.y) * (NB * NB);
+    blk::for_each(acc, [&](int r, int c, double v) { p[r * NB + c] = v; });
+}
+
+__global__ __launch_bounds__(THREADS) void k_row_products_subtract(const double *__restrict__ part, int shares, double *__restrict__ S, long lds)
+{
+    int i, j;
+    triangle_tile(blockIdx.x, i, j);
+    const double *p = part + static_cast<long>(blockIdx.x) * shares * (NB * NB);
+    for (int e = threadIdx.x; e < NB * NB; e += THREADS)
+    {
+        double s = 0.0;
+        for (int q = 0; q < shares; q++)
+            s += p[static_cast<long>(q) * (NB * NB) + e];
+        const long r = static_cast<long>(NB) * i + (e >> 6), c = static_cast<long>(NB) * j + (e & 63);
+        const double v = S[r * lds + c] - s;
+        S[r * lds + c] = v;
+        if (i != j)
+            S[c * lds + r] = v;
+    }
+}
+
 }  // namespace
 
 long flow_counters(int nb, int ne) { return 1 + (static_cast<long>(nb) + ne) * (1 + nb); }
@@ -599,23 +674,51 @@ void flow_cholesky(hipStream_t s, const FlowCall &f, int cus)
     require(f.ne == 0 || (f.X != nullptr && reinterpret_cast<uintptr_t>(f.X) % 16 == 0), "flow_cholesky: bad rows below the matrix");
     require(reinterpret_cast<uintptr_t>(f.A) % 16 == 0 && reinterpret_cast<uintptr_t>(f.Winv) % 16 == 0,
             "flow_cholesky: operands must be 16-byte aligned");
-    long tasks = 1;
+    require(!f.solve || f.ne > 0, "flow_cholesky: nothing to solve");
+    const long counters = flow_counters(f.nb, f.ne);
+    FlowArgs a{ f.A, f.lda, f.X, f.nb, f.ne, f.nu, f.solve ? 1 : 0, f.Winv, f.info, f.counters, f.counters + 1, f.counters + 1 + f.nb + f.ne, 0 };
+    long tasks = f.solve ? 0 : 1;
     for (int j = 0; j < f.nb; j++)
     {
         long u0;
         int updates;
-        column_updates(f.nb, f.ne, f.nu, j, &u0, &updates);
-        tasks += column_tiles(f.nb, f.ne, f.nu, j) + updates;
+        column_updates(a, j, &u0, &updates);
+        tasks += column_tiles(a, j) + updates;
     }
     // every running workgroup may add one number past the last task
     require(tasks < (1L << 30), "flow_cholesky: too many tiles");
-    const long counters = flow_counters(f.nb, f.ne);
-    const FlowArgs a{ f.A, f.lda, f.X, f.nb, f.ne, f.nu, f.Winv, f.info, f.counters, f.counters + 1, f.counters + 1 + f.nb + f.ne,
-                      static_cast<int>(tasks) };
+    a.tasks = static_cast<int>(tasks);
     hipLaunchKernelGGL(k_flow_init, dim3(static_cast<unsigned>(ceil_div(counters, THREADS))), dim3(THREADS), 0, s, a, counters);
     GP_CHECK_LAUNCH();
     const long wgs = std::min<long>(tasks, 2L * cus);  // two workgroups' LDS fit a CU
-    hipLaunchKernelGGL(k_flow, dim3(static_cast<unsigned>(wgs)), dim3(THREADS), 0, s, a);
+    if (f.solve)
+        hipLaunchKernelGGL(k_flow<true>, dim3(static_cast<unsigned>(wgs)), dim3(THREADS), 0, s, a);
+    else
+        hipLaunchKernelGGL(k_flow<false>, dim3(static_cast<unsigned>(wgs)), dim3(THREADS), 0, s, a);
+    GP_CHECK_LAUNCH();
+}
+
+static int row_product_shares(int n, int m)
+{
+    const long tiles = static_cast<long>(m / NB) * (m / NB + 1) / 2;
+    return static_cast<int>(std::clamp<long>(512 / tiles, 1, ceil_div(n / NB, 4)));
+}
+
+long row_products_scratch(int n, int m)
+{
+    return static_cast<long>(m / NB) * (m / NB + 1) / 2 * row_product_shares(n, m) * NB * NB;
+}
+
+void subtract_row_products(hipStream_t s, const double *V, long ldv, int n, double *S, long lds, int m, double *part)
+{
+    require(n > 0 && n % NB == 0 && m > 0 && m % NB == 0 && ldv % 2 == 0 && ldv >= n && lds >= m, "subtract_row_products: bad shape");
+    require(reinterpret_cast<uintptr_t>(V) % 16 == 0, "subtract_row_products: operand must be 16-byte aligned");
+    const int shares = row_product_shares(n, m);
+    const long tiles = static_cast<long>(m / NB) * (m / NB + 1) / 2;
+    require(tiles < (1L << 24), "subtract_row_products: too many rows");
+    hipLaunchKernelGGL(k_row_products, dim3(static_cast<unsigned>(tiles), shares), dim3(THREADS), 0, s, V, ldv, n / NB, part);
+    GP_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_row_products_subtract, dim3(static_cast<unsigned>(tiles)), dim3(THREADS), 0, s, part, shares, S, lds);
     GP_CHECK_LAUNCH();
 }
 

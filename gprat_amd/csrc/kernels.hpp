@@ -303,7 +303,8 @@ constexpr int FLOW_PANEL = 8;
 // leave as X L^-T (rows are independent, so what unused ones hold does not
 // matter); the first nu of them start as the identity's first nu block rows
 // instead (X is not read; the blocks left of a row's first nonzero one are not
-// written). The row-major inverses of L's 64x64 diagonal blocks
+// written). solve: A holds the factor and Winv its blocks' inverses already;
+// only the rows of X are computed. The row-major inverses of L's 64x64 diagonal blocks
 // go to Winv. counters: flow_counters(nb, ne) ints; info: the smallest
 // non-positive pivot's column, INT_MAX or FLOW_STALLED (both device memory,
 // set by the call). cus: the device's compute units.
@@ -313,6 +314,7 @@ struct FlowCall
     long lda;
     double *X;
     int nb, ne, nu;
+    bool solve;
     double *Winv;
     int *info, *counters;
 };
@@ -326,6 +328,18 @@ void flow_cholesky(hipStream_t s, const FlowCall &f, int cus);
 long flow_gradient_tiles(int n_pad);
 void flow_gradient(hipStream_t s, const double *WT, long ldw, int n_pad, const double *x, const double *alpha, int r, SEK sek, double sig_l,
                    double sig_v, int n, double *part, double *out);
+
+// S -= V V^T for m (a multiple of 64) rows V of n values (a multiple of 64, row
+// stride ldv); S symmetric, m x m. part: row_products_scratch(n, m) doubles.
+long row_products_scratch(int n, int m);
+void subtract_row_products(hipStream_t s, const double *V, long ldv, int n, double *S, long lds, int m, double *part);
+
+// ---- few right-hand sides (k_few.hip) -------------------------------------
+
+// V = X L^-T for `rows` (a multiple of 16) rows X of n values, stepping
+// through L (n x n) in width-wide panels with their k-major inverses Wpanel
+// (panel_inverses()); X is overwritten. X and V have row stride ldx.
+void few_rows_solve(hipStream_t s, const double *L, long lda, const double *Wpanel, int width, int n, double *X, double *V, long ldx, int rows);
 
 // Block steps of the vector solves with the saved diagonal-block inverses
 // Winv (block J at Winv + J*64*64). Forward: out[J] = W_JJ rhs[J],

@@ -97,3 +97,25 @@ def test_first_failing_pivot(ctx, column):
     with pytest.raises(capi.GpratError, match=f"at column {column}\\)"):
         ctx.cholesky(u, (0.3, 1.0, -1e-3), 1, n, r)
     assert ctx.cholesky(u, (0.3, 1.0, 1e-3), 1, n, r).shape == (1, n, n)
+
+
+@pytest.mark.parametrize("n", [100, 769, 2049, 2500])
+@pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64, 65, 200, 1100])
+def test_forward_solves_agree(ctx, n, m):
+    """Few-row kernels (0), one launch (1) and the blocked solve (2)."""
+    x, y, z = datagen.gp_problem(n, m, 8)
+    model = ctx.fit(x, y, n, 8, (1.0, 1.0, 0.1))
+    out = {}
+    try:
+        for how in "012":
+            os.environ["GPRAT_FORWARD_SOLVE"] = how
+            mean, var = model.predict(z, m)
+            out[how] = mean, var, model.predict_full_cov(z, m)[1]
+    finally:
+        del os.environ["GPRAT_FORWARD_SOLVE"]
+        model.release()
+    for how in "01":
+        assert np.array_equal(out[how][0], out["2"][0])
+        assert norm_rel(out[how][1], out["2"][1]) < TOL
+        assert norm_rel(out[how][2].ravel(), out["2"][2].ravel()) < TOL
+        assert np.array_equal(out[how][2], out[how][2].T)
