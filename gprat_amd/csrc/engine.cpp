@@ -1952,6 +1952,10 @@ void model_gradient(Model &m, const int trainable[3], double *loss_out, double g
         g.k_from_tile = true;
         g.set = true;
         g.role = k::GemmRole::Inverse;
+        DevBuf<int> queue(c, 1);
+        k::set_int(c.main, queue.get(), 0);
+        g.queue = queue.get();
+        g.max_wgs = 2 * c.cus;
         k::gemm_f64(c.main, g);
     }
     W.reset();

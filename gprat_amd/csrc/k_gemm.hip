@@ -201,12 +201,19 @@ void gemm_f64(hipStream_t s, const GemmArgs &g)
     }
     if (g.max_wgs > 0 && g.max_wgs < tiles)
     {
-        // only the trailing update runs capped
-        require(g.a_trans && !g.b_trans && g.role == GemmRole::TrailingT, "gemm_f64: capped launch for this role");
+        // the trailing update (a capped grid beside the panel stream) and
+        // W^T W: its tiles' K ranges differ, and a plain grid of the square
+        // gives each XCD the same columns of every row, so XCDs finish up to a
+        // sixth apart (CUs 75 % busy at n = 16384; 30.5 -> 24.9 ms)
+        require(g.a_trans && !g.b_trans && (g.role == GemmRole::TrailingT || g.role == GemmRole::Inverse), "gemm_f64: capped launch for this role");
         require(tiles < (1L << 30), "gemm_f64: too many tiles");
         p.queue = g.queue;
         p.tiles = static_cast<int>(tiles);
-        hipLaunchKernelGGL((k_gemm_f64_capped<true, false, 5>), dim3(static_cast<unsigned>(g.max_wgs)), dim3(THREADS), 0, s, p);
+        const dim3 wgs(static_cast<unsigned>(g.max_wgs));
+        if (g.role == GemmRole::TrailingT)
+            hipLaunchKernelGGL((k_gemm_f64_capped<true, false, 5>), wgs, dim3(THREADS), 0, s, p);
+        else
+            hipLaunchKernelGGL((k_gemm_f64_capped<true, false, 3>), wgs, dim3(THREADS), 0, s, p);
         GP_CHECK_LAUNCH();
         return;
     }
