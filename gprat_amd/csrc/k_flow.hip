@@ -650,17 +650,22 @@ __global__ __launch_bounds__(THREADS) void k_row_products_subtract(const double 
     int i, j;
     triangle_tile(blockIdx.x, i, j);
     const double *p = part + static_cast<long>(blockIdx.x) * shares * (NB * NB);
-    for (int e = threadIdx.x; e < NB * NB; e += THREADS)
-    {
-        double s = 0.0;
-        for (int q = 0; q < shares; q++)
-            s += p[static_cast<long>(q) * (NB * NB) + e];
-        const long r = static_cast<long>(NB) * i + (e >> 6), c = static_cast<long>(NB) * j + (e & 63);
-        const double v = S[r * lds + c] - s;
-        S[r * lds + c] = v;
-        if (i != j)
-            S[c * lds + r] = v;
-    }
+    const int e = blockIdx.y * THREADS + threadIdx.x;
+    double s = 0.0;
+#pragma unroll 4
+    for (int q = 0; q < shares; q++)
+        s += p[static_cast<long>(q) * (NB * NB) + e];
+    const long r = static_cast<long>(NB) * i + (e >> 6), c = static_cast<long>(NB) * j + (e & 63);
+    const double v = S[r * lds + c] - s;
+    S[r * lds + c] = v;
+    if (i != j)
+        S[c * lds + r] = v;
+}
+
+__global__ __launch_bounds__(THREADS) void k_pack_square(const double *__restrict__ S, long lds, int n, double *__restrict__ out)
+{
+    for (int c = threadIdx.x; c < n; c += THREADS)
+        out[static_cast<long>(blockIdx.x) * n + c] = S[blockIdx.x * lds + c];
 }
 
 }  // namespace
@@ -718,7 +723,14 @@ void subtract_row_products(hipStream_t s, const double *V, long ldv, int n, doub
     require(tiles < (1L << 24), "subtract_row_products: too many rows");
     hipLaunchKernelGGL(k_row_products, dim3(static_cast<unsigned>(tiles), shares), dim3(THREADS), 0, s, V, ldv, n / NB, part);
     GP_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_row_products_subtract, dim3(static_cast<unsigned>(tiles)), dim3(THREADS), 0, s, part, shares, S, lds);
+    hipLaunchKernelGGL(k_row_products_subtract, dim3(static_cast<unsigned>(tiles), NB * NB / THREADS), dim3(THREADS), 0, s, part, shares, S, lds);
+    GP_CHECK_LAUNCH();
+}
+
+void pack_square(hipStream_t s, const double *S, long lds, int n, double *out)
+{
+    require(n >= 1 && lds >= n, "pack_square: bad shape");
+    hipLaunchKernelGGL(k_pack_square, dim3(static_cast<unsigned>(n)), dim3(THREADS), 0, s, S, lds, n, out);
     GP_CHECK_LAUNCH();
 }
 

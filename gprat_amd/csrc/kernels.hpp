@@ -334,6 +334,9 @@ void flow_gradient(hipStream_t s, const double *WT, long ldw, int n_pad, const d
 long row_products_scratch(int n, int m);
 void subtract_row_products(hipStream_t s, const double *V, long ldv, int n, double *S, long lds, int m, double *part);
 
+// out[i * n + j] = S[i * lds + j] for i, j < n.
+void pack_square(hipStream_t s, const double *S, long lds, int n, double *out);
+
 // ---- few right-hand sides (k_few.hip) -------------------------------------
 
 // V = X L^-T for `rows` (a multiple of 16) rows X of n values, stepping
