@@ -231,7 +231,12 @@ __device__ __noinline__ void task_heads(const PanelArgs &a, int i, int j, double
     blk::sub_acc(blockA(a, i, j), h.lda, acc, i == j);
 }
 
-__global__ __launch_bounds__(THREADS) void k_panel_tasks(PanelArgs a)
+// Three wavefronts per SIMD's registers (170 a lane; every kernel that calls the
+// tasks says so, or they are compiled without a bound): a workgroup has to fit
+// the hole that one workgroup of the trailing update (212 a lane) leaves. With
+// 260 a launch of the panel stream waited for a whole update, 4.9 ms at
+// n = 16384, and the fit and prediction there took 54.4 ms.
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_panel_tasks(PanelArgs a)
 {
     __shared__ alignas(16) double buf0[NB * blk::XS];
     __shared__ alignas(16) double buf1[NB * blk::XS];
@@ -284,7 +289,7 @@ __device__ __forceinline__ PanelArgs panel_of(const InverseArgs &g, int panel)
     return a;
 }
 
-__global__ __launch_bounds__(THREADS) void k_inverse_place(InverseArgs g)
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_inverse_place(InverseArgs g)
 {
     __shared__ alignas(16) double buf0[NB * blk::XS];
     const int per = g.width / NB;
@@ -293,7 +298,7 @@ __global__ __launch_bounds__(THREADS) void k_inverse_place(InverseArgs g)
 
 // Doubling level h of every panel (grid: block (rb, cb) of the pair, pair,
 // panel): the whole join at h = 1, one of its two phases above.
-__global__ __launch_bounds__(THREADS) void k_inverse_join(InverseArgs g, int h, int phase)
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_inverse_join(InverseArgs g, int h, int phase)
 {
     __shared__ alignas(16) double buf0[NB * blk::XS];
     __shared__ alignas(16) double buf1[NB * blk::XS];
