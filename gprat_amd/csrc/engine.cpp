@@ -524,9 +524,13 @@ void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mix
         flow(c, A, lda, n_pad, Winv, Wpanel, X ? X : A + static_cast<long>(n_pad) * lda, extra, unit);
         return;
     }
-    require(X == nullptr && unit == 0, "cholesky: the panel schedule takes its rows below the matrix");
+    require(X == nullptr, "cholesky: the panel schedule takes its rows below the matrix");
+    require(unit >= 0 && unit <= n_pad && unit <= extra && unit % 64 == 0, "cholesky: bad identity rows");
     // rows of L and the rows below it that ride along (right-hand sides)
     const long rows = static_cast<long>(n_pad) + extra;
+    // those that panels up to column pe concern (identity rows come last and
+    // start in their own column)
+    auto rows_to = [&](int pe) { return static_cast<long>(n_pad) + (extra - unit) + std::min(unit, pe); };
     const bool ahead = use_lookahead() && c.panel != c.main;
     hipStream_t T = ahead ? c.trail : c.main, P = ahead ? c.panel : c.main;
     // Two trailing workgroups per CU, minus the reserve. The FP32 product
@@ -630,7 +634,7 @@ void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mix
     auto rows_below = [&](int p0, int pe, hipEvent_t solved)
     {
         Timed t(c, T, "panel_rows");
-        const int w = pe - p0, R = static_cast<int>(rows - pe);
+        const int w = pe - p0, R = static_cast<int>(rows_to(pe) - pe);
         double *panel = A + static_cast<long>(pe) * lda + p0;
         k::rows_solve(T, A, lda, pe, p0, R, w, Wblock(p0), Bo, Xs.get(), w);
         wait(T, solved, P);
@@ -646,7 +650,7 @@ void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mix
     {
         Timed t(c, T, "syrk_trailing");
         double *C = A + static_cast<long>(q1) * lda + pe;
-        const int M = static_cast<int>(rows - q1), N = n_pad - pe, K = pe - p0;
+        const int M = static_cast<int>(rows_to(pe) - q1), N = n_pad - pe, K = pe - p0;
         if (mixed)
             k::gemm_f32_trailing(T, p32.get(), rows, q1 - pe, 0, C, lda, M, N, K, q1 - pe, cap, queues.get() + p0 / Bo);
         else
@@ -673,7 +677,7 @@ void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mix
             wait(T, factored, P);
             rows_below(p0, pe, solved);
             trailed = nullptr;
-            if (q1 < rows)
+            if (q1 < rows_to(pe))
             {
                 trailing(p0, pe, q1);
                 trailed = record(T);
@@ -1177,7 +1181,7 @@ void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int
     m.fp32_updates = precision == GPRAT_PRECISION_MIXED && !one_launch(m.n_pad, true);
     const std::size_t xl = static_cast<std::size_t>(n) + r - 1;
     m.x = DevBuf<double>(c, xl);
-    m.L = DevBuf<double>(c, static_cast<std::size_t>(m.n_pad) * m.lda);
+    m.L = DevBuf<double>(c, (static_cast<std::size_t>(m.n_pad) + (riding.X ? 0 : riding.extra)) * m.lda);
     m.Winv = DevBuf<double>(c, static_cast<std::size_t>(m.n_pad) * 64);
     m.wblock = panel_width(m.n_pad);
     if (keep_inverses)
@@ -1187,6 +1191,8 @@ void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int
         Timed t(c, c.main, "assemble");
         k::assemble_lower(c.main, m.x.get(), r, m.sek, m.L.get(), m.lda, n, m.n_pad);
     }
+    if (riding.fill)
+        riding.fill(m.L.get() + static_cast<long>(m.n_pad) * m.lda);
     cholesky(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), precision == GPRAT_PRECISION_MIXED, m.Wpanel.get(),
              riding.extra, riding.X, riding.unit);
     if (m.fp32_updates)
@@ -1844,6 +1850,31 @@ static void gradient_results(const Model &m, const double *t, const double *sums
     grad[2] = trainable[2] ? sigmoid(to_unconstrained(m.sek.noise, true)) * (0.5 / Nn * (sums[4] - t[2])) : 0.0;
 }
 
+// Kinv (lower) = W^T W for lower triangular W (row-major, n_pad x n_pad, both
+// with row stride lda), the tiles from a device counter.
+static void inverse_product(Context &c, const double *W, long lda, int n_pad, double *Kinv)
+{
+    k::GemmArgs g{};
+    g.A = W;
+    g.lda = lda;
+    g.B = W;
+    g.ldb = lda;
+    g.C = Kinv;
+    g.ldc = lda;
+    g.M = g.N = g.K = n_pad;
+    g.a_trans = true;
+    g.b_trans = false;
+    g.lower = true;
+    g.k_from_tile = true;
+    g.set = true;
+    g.role = k::GemmRole::Inverse;
+    DevBuf<int> queue(c, 1);
+    k::set_int(c.main, queue.get(), 0);
+    g.queue = queue.get();
+    g.max_wgs = 2 * c.cus;
+    k::gemm_f64(c.main, g);
+}
+
 // Loss and softplus-space gradient at theta. K^-1 is formed as W^T W with
 // W = L^-1, n^3 flops in total instead of the reference's explicit 2 n^3
 // double solve (core/src/cpu/gp_functions.cpp:953-966); the trace and quadratic
@@ -1852,7 +1883,10 @@ static void gradient_results(const Model &m, const double *t, const double *sums
 // rows that ride along, and reduce each tile of K^-1 where it is formed
 // (measured on MI355X, with the blocked solve on the panel schedule's
 // factor / so: n = 1024 1.42 / 0.45 ms, 4096 6.5 / 2.8, 8192 20.0 / 13.9, 12288
-// 48.3 / 45.2); larger ones fit a model and use model_gradient().
+// 48.3 / 45.2); larger ones on the
+// panel schedule, whose trailing updates carry the identity rows where the
+// diagonal-block chain would leave the device idle (n = 16384 89.6 -> 81.8 ms),
+// and form K^-1 from a k-major copy with 128x128 tiles.
 void loss_gradient(Context &c,
                    const double *x,
                    std::size_t x_len,
@@ -1867,7 +1901,7 @@ void loss_gradient(Context &c,
 {
     Model m;
     const int n_pad = static_cast<int>(padded(n));
-    if (!(trainable[0] || trainable[1] || trainable[2]) || !one_launch(n_pad, false))
+    if (!(trainable[0] || trainable[1] || trainable[2]))
     {
         fit(c, m, x, x_len, y, y_len, n, r, theta, GPRAT_PRECISION_FP64);
         model_gradient(m, trainable, loss_out, grad);
@@ -1878,25 +1912,66 @@ void loss_gradient(Context &c,
     require(y != nullptr && y_len >= static_cast<std::size_t>(n), "training output must hold n values");
     check_training(x, x_len, n, r, theta, GPRAT_PRECISION_FP64);
     c.make_current();
+    const bool flow = one_launch(n_pad, false);
     const long lda = leading_dim(n_pad);
-    DevBuf<double> X(c, static_cast<std::size_t>(n_pad + 64) * lda);
-    double *z = X.get() + static_cast<long>(n_pad) * lda;
+    const int extra = n_pad + 64;
+    DevBuf<double> X;
     m.y = DevBuf<double>(c, n_pad);
     k::fill(c.main, m.y.get(), n_pad, 0.0);
     upload(c, m.y.get(), y, static_cast<std::size_t>(n));
-    GP_HIP(hipMemcpyAsync(z, m.y.get(), sizeof(double) * n_pad, hipMemcpyDeviceToDevice, c.main));
-    factor(c, m, x, x_len, n, r, theta, GPRAT_PRECISION_FP64, { X.get(), n_pad + 64, n_pad }, false);
+    double *z = nullptr, *WT = nullptr;
+    auto targets = [&] { GP_HIP(hipMemcpyAsync(z, m.y.get(), sizeof(double) * n_pad, hipMemcpyDeviceToDevice, c.main)); };
+    Riding riding;
+    riding.extra = extra;
+    riding.unit = n_pad;
+    if (flow)
+    {
+        // the launch makes the identity itself, and its rows come first
+        X = DevBuf<double>(c, static_cast<std::size_t>(extra) * lda);
+        riding.X = WT = X.get();
+        z = WT + static_cast<long>(n_pad) * lda;
+        targets();
+    }
+    else
+        riding.fill = [&](double *below)
+        {
+            z = below;
+            WT = below + 64L * lda;
+            k::fill(c.main, below, static_cast<long>(extra) * lda, 0.0);
+            targets();
+            k::set_diagonal(c.main, WT, lda, n_pad, 1.0);
+        };
+    factor(c, m, x, x_len, n, r, theta, GPRAT_PRECISION_FP64, riding, false);
     m.alpha = DevBuf<double>(c, n_pad);
     {
         Timed t(c, c.main, "solve");
-        k::rowdot(c.main, X.get(), lda, n_pad, n_pad, z, m.alpha.get(), false, true);
+        k::rowdot(c.main, WT, lda, n_pad, n_pad, z, m.alpha.get(), false, true);
     }
     k::loss_terms(c.main, m.L.get(), m.lda, m.y.get(), m.alpha.get(), m.n, c.scalars.get());
+    const double sig_l = sigmoid(to_unconstrained(m.sek.lengthscale, false));
+    const double sig_v = sigmoid(to_unconstrained(m.sek.vertical, false));
     DevBuf<double> part(c, static_cast<std::size_t>(k::flow_gradient_tiles(n_pad)) * 5);
+    if (flow)
     {
         Timed t(c, c.main, "gradient");
-        k::flow_gradient(c.main, X.get(), lda, n_pad, m.x.get(), m.alpha.get(), r, m.sek, sigmoid(to_unconstrained(m.sek.lengthscale, false)),
-                         sigmoid(to_unconstrained(m.sek.vertical, false)), n, part.get(), c.scalars.get() + 8);
+        k::flow_gradient(c.main, WT, lda, n_pad, m.x.get(), m.alpha.get(), r, m.sek, sig_l, sig_v, n, part.get(), c.scalars.get() + 8);
+    }
+    else
+    {
+        {
+            // the product's operands are k-major; K^-1 takes the factor's place
+            Timed t(c, c.main, "inverse");
+            DevBuf<double> W(c, static_cast<std::size_t>(n_pad) * lda);
+            const int width = panel_width(n_pad);
+            for (int p0 = 0; p0 < n_pad; p0 += width)
+            {
+                const int w = std::min(width, n_pad - p0);
+                k::panel_to_f64t(c.main, WT, lda, 0, p0, p0 + w, w, W.get() + static_cast<long>(p0) * lda, lda);
+            }
+            inverse_product(c, W.get(), lda, n_pad, m.L.get());
+        }
+        Timed t(c, c.main, "gradient");
+        k::gradient_sums(c.main, m.L.get(), lda, m.x.get(), m.alpha.get(), r, m.sek, sig_l, sig_v, n, part.get(), c.scalars.get() + 8);
     }
     double h[13];
     GP_HIP(hipMemcpyAsync(h, c.scalars.get(), sizeof h, hipMemcpyDefault, c.main));
@@ -1951,25 +2026,7 @@ void model_gradient(Model &m, const int trainable[3], double *loss_out, double g
         Timed tm(c, c.main, "inverse");
         trsm_blocked(c, m.L.get(), m.lda, m.Winv.get(), m.Wpanel.get(), m.wblock, m.n_pad, Kinv.get(), m.lda, m.n_pad, true, W.get(),
                      m.lda);
-        k::GemmArgs g{};
-        g.A = W.get();
-        g.lda = m.lda;
-        g.B = W.get();
-        g.ldb = m.lda;
-        g.C = Kinv.get();
-        g.ldc = m.lda;
-        g.M = g.N = g.K = m.n_pad;
-        g.a_trans = true;
-        g.b_trans = false;
-        g.lower = true;
-        g.k_from_tile = true;
-        g.set = true;
-        g.role = k::GemmRole::Inverse;
-        DevBuf<int> queue(c, 1);
-        k::set_int(c.main, queue.get(), 0);
-        g.queue = queue.get();
-        g.max_wgs = 2 * c.cus;
-        k::gemm_f64(c.main, g);
+        inverse_product(c, W.get(), m.lda, m.n_pad, Kinv.get());
     }
     W.reset();
     DevBuf<double> part(c, static_cast<std::size_t>(k::grad_tiles(n)) * 5);

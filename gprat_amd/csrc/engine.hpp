@@ -269,9 +269,9 @@ void cholesky_fp64(Context &c, double *A, long lda, int n_pad, double *Winv);
 // extra: rows below the n_pad x n_pad matrix (A holds n_pad + extra rows)
 // that the factorisation treats as rows of L below it: on return they hold
 // B L^-T for the B they held (the forward solve of their transposes).
-// Their rows start at X (row stride lda; null: right below A); the first
-// `unit` of them are identity rows that need not be stored (both
-// one_launch() sizes only). The factor is
+// Their rows start at X (row stride lda; null: right below A). `unit` of them
+// are the identity's first rows: the first ones for one_launch() sizes, which
+// need not be stored, else the last ones. The factor is
 // complete in stream order on c.main; c.sync() and check_pivots() report a
 // pivot that was not positive.
 void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel = nullptr, int extra = 0, double *X = nullptr,
@@ -288,11 +288,13 @@ void solve_spd(Context &c, const double *L, long lda, const double *Winv, int n_
 void trsm_blocked(Context &c, const double *L, long lda, const double *Winv, const double *Wpanel, int wblock, int n_pad, double *B,
                   long ldb, int ncols, bool tri_rhs, double *out, long ldo);
 
-// Rows that ride along in a factorisation (cholesky(), one_launch() sizes).
+// Rows that ride along in a factorisation (cholesky()): in X for one_launch()
+// sizes, else right below the matrix, where `fill` writes them.
 struct Riding
 {
     double *X = nullptr;
     int extra = 0, unit = 0;
+    std::function<void(double *)> fill;
 };
 // keep_inverses: the panels' whole inverses, which the solves step through,
 // are wanted. Pivots as cholesky().
