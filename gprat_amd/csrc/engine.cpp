@@ -453,23 +453,28 @@ const Context::PanelPlanDev &Context::cached_plan(long key, const std::function<
 // step k-1's update has reached it) and factors that block, while the
 // `trail` stream solves panel k's rows and applies panel k to everything
 // below block k+1.
-// Sizes the dataflow launch factors faster than the panel schedule.
-// Measured on MI355X (whole FP64 fit, panels / dataflow, ms): n = 1024
-// 0.82 / 0.42, 4096 3.58 / 2.01, 8192 9.26 / 6.45, 10240 13.6 / 11.1, 12288
-// 19.7 / 18.3, 14336 27.2 / 28.3, 16384 36.9 / 42.0: beyond, its 64x64 tiles
-// reuse an operand too little. A mixed-precision fit whose whole factor is
-// FP64 on this path is faster than with FP32 trailing updates up to n = 10240
-// (2048 2.09 / 1.07, 8192 9.8 / 7.1, 10240 13.2 / 11.9, 12288 16.9 / 19.3).
-// GPRAT_FLOW_LIMIT overrides, and the panel
-// schedule's own overrides ask for that schedule.
-constexpr int FLOW_LIMIT = 12288, FLOW_LIMIT_MIXED = 10240;
-bool one_launch(int n_pad, bool mixed)
+// Whether the dataflow launch is faster than the panel schedule. Its 64x64
+// tiles run at 33 TF/s where the panels' 128x128 tiles reach 58, but each 64
+// columns cost it 15 us of chain and the panels 60 to 70, so the line is where
+// the work per column, n (n / 3 + rows that ride along; identity rows
+// average a third), outgrows the difference. Measured on MI355X (panels /
+// dataflow, ms):
+//   fit       n = 1024 0.80 / 0.39, 4096 3.5 / 1.9, 8192 8.9 / 6.4, 10240 12.7 / 11.0, 12288 18.3 / 18.4
+//   one call  n = 6144 m = 1536 6.4 / 4.6, m = 6144 8.8 / 9.1; n = 8192 m = 2048 10.4 / 9.6, m = 8192 16.7 / 21.0;
+//             n = 10240 m = 640 13.2 / 12.4, m = 2560 16.2 / 17.7
+//   gradient  n = 4096 4.8 / 2.8, 8192 14.9 / 13.9, 10240 23.9 / 26.4
+//   mixed fit n = 4096 4.1 / 2.3, 8192 10.0 / 7.1, 10240 13.7 / 12.0, 12288 16.9 / 19.3
+// (in a mixed fit the whole factor is then FP64; the FP32 updates it replaces
+// are faster, hence the lower line). GPRAT_FLOW_LIMIT (a largest n) overrides,
+// and the panel schedule's own overrides ask for that schedule.
+bool one_launch(int n_pad, bool mixed, int extra, int unit)
 {
     if (std::getenv("GPRAT_CHOLESKY_BLOCK") || std::getenv("GPRAT_LOOKAHEAD"))
         return false;
     if (const char *e = std::getenv("GPRAT_FLOW_LIMIT"))
         return n_pad <= std::atoi(e);
-    return n_pad <= (mixed ? FLOW_LIMIT_MIXED : FLOW_LIMIT);
+    const double work = static_cast<double>(n_pad) * (n_pad / 3.0 + (extra - unit) + unit / 3.0);
+    return work <= (mixed ? 4.2e7 : 4.8e7);
 }
 
 void check_pivots(Context &c)
@@ -519,7 +524,7 @@ void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mix
 {
     require(n_pad % 128 == 0 && lda >= n_pad && lda % 2 == 0, "cholesky: bad layout");
     require(extra >= 0 && extra % 64 == 0, "cholesky: extra rows must come in 64s");
-    if (one_launch(n_pad, mixed))
+    if (one_launch(n_pad, mixed, extra, unit))
     {
         flow(c, A, lda, n_pad, Winv, Wpanel, X ? X : A + static_cast<long>(n_pad) * lda, extra, unit);
         return;
@@ -1178,7 +1183,7 @@ void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int
     m.lda = leading_dim(m.n_pad);
     m.sek = SEK{ theta[0], theta[1], theta[2] };
     m.precision = precision;
-    m.fp32_updates = precision == GPRAT_PRECISION_MIXED && !one_launch(m.n_pad, true);
+    m.fp32_updates = precision == GPRAT_PRECISION_MIXED && !one_launch(m.n_pad, true, riding.extra, riding.unit);
     const std::size_t xl = static_cast<std::size_t>(n) + r - 1;
     m.x = DevBuf<double>(c, xl);
     m.L = DevBuf<double>(c, (static_cast<std::size_t>(m.n_pad) + (riding.X ? 0 : riding.extra)) * m.lda);
@@ -1277,7 +1282,7 @@ void fit(Context &c,
     k::fill(c.main, m.y.get(), n_pad, 0.0);
     upload(c, m.y.get(), y, static_cast<std::size_t>(n));
     DevBuf<double> rhs;
-    if (one_launch(n_pad, mixed))
+    if (one_launch(n_pad, mixed, 64))
     {
         // the targets ride along as a row below the matrix: z = L^-1 y
         rhs = DevBuf<double>(c, static_cast<std::size_t>(64) * leading_dim(n_pad));
@@ -1882,8 +1887,7 @@ static void inverse_product(Context &c, const double *W, long lda, int n_pad, do
 // triangle of K^-1. Sizes that factor in one launch take W^T from identity
 // rows that ride along, and reduce each tile of K^-1 where it is formed
 // (measured on MI355X, with the blocked solve on the panel schedule's
-// factor / so: n = 1024 1.42 / 0.45 ms, 4096 6.5 / 2.8, 8192 20.0 / 13.9, 12288
-// 48.3 / 45.2); larger ones on the
+// factor / so: n = 1024 1.42 / 0.45 ms, 4096 6.5 / 2.8, 8192 20.0 / 13.9); larger ones on the
 // panel schedule, whose trailing updates carry the identity rows where the
 // diagonal-block chain would leave the device idle (n = 16384 89.6 -> 81.8 ms),
 // and form K^-1 from a k-major copy with 128x128 tiles.
@@ -1912,9 +1916,9 @@ void loss_gradient(Context &c,
     require(y != nullptr && y_len >= static_cast<std::size_t>(n), "training output must hold n values");
     check_training(x, x_len, n, r, theta, GPRAT_PRECISION_FP64);
     c.make_current();
-    const bool flow = one_launch(n_pad, false);
-    const long lda = leading_dim(n_pad);
     const int extra = n_pad + 64;
+    const bool flow = one_launch(n_pad, false, extra, n_pad);
+    const long lda = leading_dim(n_pad);
     DevBuf<double> X;
     m.y = DevBuf<double>(c, n_pad);
     k::fill(c.main, m.y.get(), n_pad, 0.0);
@@ -1996,7 +2000,7 @@ void model_gradient(Model &m, const int trainable[3], double *loss_out, double g
     const double sig_l = sigmoid(to_unconstrained(m.sek.lengthscale, false));
     const double sig_v = sigmoid(to_unconstrained(m.sek.vertical, false));
     double sums[5];
-    if (one_launch(m.n_pad, false))
+    if (one_launch(m.n_pad, false, m.n_pad, m.n_pad))
     {
         DevBuf<double> X(c, static_cast<std::size_t>(m.n_pad) * m.lda), part(c, static_cast<std::size_t>(k::flow_gradient_tiles(m.n_pad)) * 5);
         {

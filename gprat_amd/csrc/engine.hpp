@@ -280,8 +280,9 @@ void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mix
 // not positive.
 void check_pivots(Context &c);
 int panel_width(int n_pad);
-// The factorisation of this size runs as one dataflow launch (k_flow.hip).
-bool one_launch(int n_pad, bool mixed);
+// The factorisation of this size, with `extra` rows riding along, `unit` of them
+// identity rows, runs as one dataflow launch (k_flow.hip).
+bool one_launch(int n_pad, bool mixed, int extra = 0, int unit = 0);
 void refine_alpha(Model &m, double *work);
 void solve_spd(Context &c, const double *L, long lda, const double *Winv, int n_pad, const double *y, double *work, double *out,
                const double *Wpanel = nullptr, int wblock = 0);
