@@ -269,6 +269,7 @@ int gprat_cholesky(gprat_context *ctx,
             const Tiling t = check_tiling(n_tiles, n_tile_size, 0, 0, n_reg);
             gpamd::require(tiles_out != nullptr, "tiles_out is null");
             std::lock_guard<std::recursive_mutex> g(c.mu);
+            c.begin_call();
             gpamd::Model model;
             gpamd::factor(c, model, train_in, train_in_len, t.n, n_reg, theta, GPRAT_PRECISION_FP64, {}, false);
             gpamd::cholesky_tiles(model, n_tiles, n_tile_size, tiles_out);

@@ -13,7 +13,9 @@
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
+#include <initializer_list>
 #include <numbers>
+#include <optional>
 
 namespace gpamd
 {
@@ -217,6 +219,7 @@ Context::Context(int dev, int ns) : device(dev), n_streams(ns), pool(dev)
     info = DevBuf<int>(*this, 1);
     scalars = DevBuf<double>(*this, 64);
     GP_HIP(hipHostMalloc(reinterpret_cast<void **>(&host_info), sizeof(int), hipHostMallocDefault));
+    GP_HIP(hipHostMalloc(reinterpret_cast<void **>(&stage), STAGE * sizeof(double), hipHostMallocDefault));
     k::noalloc_scratch_init(device);
 }
 
@@ -237,6 +240,8 @@ Context::~Context()
     scalars.reset();
     if (host_info)
         hipHostFree(host_info);
+    if (stage)
+        hipHostFree(stage);
     if (trail && trail != main)
         hipStreamDestroy(trail);
     if (panel && panel != main)
@@ -304,8 +309,28 @@ void Context::sync()
     if (trail != main)
         GP_HIP(hipStreamSynchronize(trail));
     GP_HIP(hipStreamSynchronize(main));
+    stage_busy = false;
     if (!pending.empty())
         resolve_profiling();
+}
+
+void Context::begin_call()
+{
+    make_current();
+    if (stage_busy)  // a call that failed left work behind
+        sync();
+    stage_used = 0;
+}
+
+double *Context::stage_take(std::size_t count)
+{
+    count = (count + 1) / 2 * 2;  // 16-byte aligned
+    if (count > STAGE - stage_used)
+        return nullptr;
+    double *p = stage + stage_used;
+    stage_used += count;
+    stage_busy = true;
+    return p;
 }
 
 // Optional timing bracket around a launch sequence.
@@ -502,7 +527,7 @@ static void flow(Context &c, double *A, long lda, int n_pad, double *Winv, doubl
         DevBuf<double> tmp(c, static_cast<std::size_t>(std::max(1L, k::panel_inverses_scratch(n_pad, width))));
         k::panel_inverses(c.main, A, lda, Winv, n_pad, width, Wpanel, tmp.get());
     }
-    GP_HIP(hipMemcpyAsync(c.host_info, c.info.get(), sizeof(int), hipMemcpyDeviceToHost, c.main));
+    k::report(c.main, nullptr, 0, nullptr, c.info.get(), c.host_info);
 }
 
 // X L^-T in place for `rows` rows X (row stride lda, as L; the first `unit`
@@ -513,7 +538,7 @@ static void flow_solve(Context &c, const double *L, long lda, int n_pad, const d
     DevBuf<int> counters(c, static_cast<std::size_t>(k::flow_counters(nb, ne)));
     k::flow_cholesky(c.main, k::FlowCall{ const_cast<double *>(L), lda, X, nb, ne, unit / 64, true, const_cast<double *>(Winv), c.info.get(), counters.get() },
                      c.cus);
-    GP_HIP(hipMemcpyAsync(c.host_info, c.info.get(), sizeof(int), hipMemcpyDeviceToHost, c.main));
+    k::report(c.main, nullptr, 0, nullptr, c.info.get(), c.host_info);
 }
 
 void cholesky_fp64(Context &c, double *A, long lda, int n_pad, double *Winv) { cholesky(c, A, lda, n_pad, Winv, false); }
@@ -697,7 +722,7 @@ void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mix
         wait(c.main, record(T), T);
         wait(c.main, record(P), P);
     }
-    GP_HIP(hipMemcpyAsync(c.host_info, c.info.get(), sizeof(int), hipMemcpyDeviceToHost, c.main));
+    k::report(c.main, nullptr, 0, nullptr, c.info.get(), c.host_info);
     c.sync();
     for (auto e : used)
         c.recycle(e);
@@ -1156,11 +1181,85 @@ static double variance_refined(Context &c, const FactorView &m, const double *z,
 // ---------------------------------------------------------------------------
 // Model operations
 
-static void upload(Context &c, double *dst, const double *src, std::size_t count)
+// Memory the host can read and write (not a device buffer of the caller's).
+static bool host_memory(const void *p)
 {
-    if (count)
-        GP_HIP(hipMemcpyAsync(dst, src, count * sizeof(double), hipMemcpyDefault, c.main));
+    hipPointerAttribute_t a{};
+    if (hipPointerGetAttributes(&a, p) != hipSuccess)
+    {
+        (void)hipGetLastError();  // plain host memory is unknown to the runtime
+        return true;
+    }
+    return a.type != hipMemoryTypeDevice;
 }
+
+// src[0 .. n) to dst, zeros up to n_pad, and the same to `also` if given.
+struct Upload
+{
+    const double *src;
+    std::size_t n;
+    double *dst;
+    std::size_t n_pad;
+    double *also = nullptr;
+};
+static void upload(Context &c, std::initializer_list<Upload> items)
+{
+    k::PlaceItem staged[3];
+    int count = 0;
+    for (const Upload &u : items)
+    {
+        if (u.n == 0 && u.n_pad == 0)
+            continue;
+        double *p = u.n < (1u << 30) && u.n_pad < (1u << 30) && host_memory(u.src) ? c.stage_take(u.n) : nullptr;
+        if (p)
+        {
+            std::memcpy(p, u.src, u.n * sizeof(double));
+            staged[count++] = { p, u.dst, u.also, static_cast<int>(u.n), static_cast<int>(u.n_pad) };
+            continue;
+        }
+        for (double *dst : { u.dst, u.also })
+        {
+            if (!dst)
+                continue;
+            if (u.n_pad > u.n)
+                k::fill(c.main, dst + u.n, static_cast<long>(u.n_pad - u.n), 0.0);
+            GP_HIP(hipMemcpyAsync(dst, u.src, u.n * sizeof(double), hipMemcpyDefault, c.main));
+        }
+    }
+    if (count)
+        k::place(c.main, staged, count);
+}
+
+// A result of `count` values on its way to the caller's memory: kernels write
+// to get(), send() goes before the call's last sync() and deliver() after it.
+class Result
+{
+  public:
+    Result(Context &c, double *user, std::size_t count) : c_(c), user_(user), count_(count)
+    {
+        if (host_memory(user))
+            staged_ = c.stage_take(count);
+        if (!staged_)
+            device_ = DevBuf<double>(c, count);
+    }
+    double *get() const { return staged_ ? staged_ : device_.get(); }
+    void send()
+    {
+        if (!staged_)
+            GP_HIP(hipMemcpyAsync(user_, device_.get(), sizeof(double) * count_, hipMemcpyDefault, c_.main));
+    }
+    void deliver() const
+    {
+        if (staged_)
+            std::memcpy(user_, staged_, sizeof(double) * count_);
+    }
+
+  private:
+    Context &c_;
+    double *user_, *staged_ = nullptr;
+    std::size_t count_;
+    DevBuf<double> device_;
+};
 
 static void check_training(const double *x, std::size_t x_len, int n, int r, const double *theta, int precision)
 {
@@ -1191,7 +1290,7 @@ void factor(Context &c, Model &m, const double *x, std::size_t x_len, int n, int
     m.wblock = panel_width(m.n_pad);
     if (keep_inverses)
         m.Wpanel = DevBuf<double>(c, static_cast<std::size_t>(ceil_div(m.n_pad, m.wblock)) * m.wblock * m.wblock);
-    upload(c, m.x.get(), x, xl);
+    upload(c, { { x, xl, m.x.get(), xl } });
     {
         Timed t(c, c.main, "assemble");
         k::assemble_lower(c.main, m.x.get(), r, m.sek, m.L.get(), m.lda, n, m.n_pad);
@@ -1277,17 +1376,12 @@ void fit(Context &c,
     check_training(x, x_len, n, r, theta, precision);
     const bool mixed = precision == GPRAT_PRECISION_MIXED;
     const int n_pad = static_cast<int>(padded(n));
-    c.make_current();
+    c.begin_call();
     m.y = DevBuf<double>(c, n_pad);
-    k::fill(c.main, m.y.get(), n_pad, 0.0);
-    upload(c, m.y.get(), y, static_cast<std::size_t>(n));
     DevBuf<double> rhs;
-    if (one_launch(n_pad, mixed, 64))
-    {
-        // the targets ride along as a row below the matrix: z = L^-1 y
+    if (one_launch(n_pad, mixed, 64))  // the targets ride along as a row below the matrix: z = L^-1 y
         rhs = DevBuf<double>(c, static_cast<std::size_t>(64) * leading_dim(n_pad));
-        GP_HIP(hipMemcpyAsync(rhs.get(), m.y.get(), sizeof(double) * n_pad, hipMemcpyDeviceToDevice, c.main));
-    }
+    upload(c, { { y, static_cast<std::size_t>(n), m.y.get(), static_cast<std::size_t>(n_pad), rhs.get() } });
     factor(c, m, x, x_len, n, r, theta, precision, { rhs.get(), rhs.get() ? 64 : 0, 0 });
     m.alpha = DevBuf<double>(c, n_pad);
     DevBuf<double> work(c, n_pad);
@@ -1420,51 +1514,48 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
     require(z != nullptr && z_len >= static_cast<std::size_t>(mt) + m.r - 1,
             "predict: test input must hold m + n_reg - 1 values");
     require(mean != nullptr, "predict: mean output is null");
-    c.make_current();
+    c.begin_call();
     const std::size_t zl = static_cast<std::size_t>(mt) + m.r - 1;
     DevBuf<double> dz(c, zl);
-    upload(c, dz.get(), z, zl);
+    upload(c, { { z, zl, dz.get(), zl } });
     const int splits = k::mean_splits(m.n, mt);
     DevBuf<double> partial(c, static_cast<std::size_t>(splits) * mt);
-    DevBuf<double> dmean(c, mt);
+    Result means(c, mean, mt);
+    std::optional<Result> vars;
+    if (var)
+        vars.emplace(c, var, mt);
     const ForwardSolve how = m.mixed ? ForwardSolve::Blocked : forward_solve(m, mt);
     // beside the row methods, whose launches leave most of the device idle,
     // the mean's kernels run on the second stream
     SideStream side(c, var && how != ForwardSolve::Blocked);
     {
         Timed t(c, side.stream(), "mean");
-        k::predict_mean(side.stream(), m.x, dz.get(), m.alpha, m.r, m.sek, m.n, mt, partial.get(), splits, dmean.get());
+        k::predict_mean(side.stream(), m.x, dz.get(), m.alpha, m.r, m.sek, m.n, mt, partial.get(), splits, means.get());
     }
     side.done();
-    DevBuf<double> dvar, rows;
+    DevBuf<double> rows;
     bool solved_here = false;  // by a dataflow launch: its completion is checked below
     if (var && m.mixed && m.refine_variance)
     {
         const int m_pad = static_cast<int>(round_up(mt, 64));
-        dvar = DevBuf<double>(c, mt);
-        const double corr = variance_refined(c, m, dz.get(), mt, m_pad, dvar.get());
+        const double corr = variance_refined(c, m, dz.get(), mt, m_pad, vars->get());
         if (m.variance_correction)
             *m.variance_correction = corr;
-        GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
     }
     else if (var && m.mixed)
     {
         const int m_pad = static_cast<int>(round_up(mt, 64));
         DevBuf<double> colsq(c, m_pad);
-        dvar = DevBuf<double>(c, mt);
         variance_colsq_f32(c, m, dz.get(), mt, m_pad, colsq.get());
-        k::variance_finish(c.main, colsq.get(), m.sek.vertical, mt, dvar.get());
-        GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
+        k::variance_finish(c.main, colsq.get(), m.sek.vertical, mt, vars->get());
     }
     else if (var && how != ForwardSolve::Blocked)
     {
         solved_here = how == ForwardSolve::OneLaunch;
         DevBuf<double> sumsq(c, mt);
-        dvar = DevBuf<double>(c, mt);
         rows = solved_rows(m, how, dz.get(), mt);
         k::row_sumsq(c.main, rows.get(), m.lda, mt, m.n_pad, sumsq.get());
-        k::variance_finish(c.main, sumsq.get(), m.sek.vertical, mt, dvar.get());
-        GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
+        k::variance_finish(c.main, sumsq.get(), m.sek.vertical, mt, vars->get());
     }
     else if (var)
     {
@@ -1472,7 +1563,6 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
         const long ldb = m_pad;
         DevBuf<double> B(c, static_cast<std::size_t>(m.n_pad) * ldb);
         DevBuf<double> colsq(c, m_pad);
-        dvar = DevBuf<double>(c, mt);
         {
             Timed t(c, c.main, "assemble");
             k::assemble_cross_t(c.main, m.x, dz.get(), m.r, m.sek, B.get(), ldb, m.n, m.n_pad, mt, m_pad);
@@ -1489,12 +1579,16 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
             }
             variance_solve<VarianceF64>(c, m.L, m.lda, m.Wpanel ? m.Wpanel : Wt.get(), NBK, m.n_pad, B.get(), m_pad, mt, colsq.get());
         }
-        k::variance_finish(c.main, colsq.get(), m.sek.vertical, mt, dvar.get());
-        GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
+        k::variance_finish(c.main, colsq.get(), m.sek.vertical, mt, vars->get());
     }
     side.join();
-    GP_HIP(hipMemcpyAsync(mean, dmean.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
+    means.send();
+    if (vars)
+        vars->send();
     c.sync();
+    means.deliver();
+    if (vars)
+        vars->deliver();
     if (solved_here)
         check_pivots(c);
 }
@@ -1531,10 +1625,10 @@ void predict_full_cov_view(const FactorView &m, const double *z, std::size_t z_l
         return;
     require(cov != nullptr, "predict_full_cov: covariance output is null");
     predict_view(m, z, z_len, mt, mean, nullptr);
-    c.make_current();
+    c.begin_call();
     const std::size_t zl = static_cast<std::size_t>(mt) + m.r - 1;
     DevBuf<double> dz(c, zl);
-    upload(c, dz.get(), z, zl);
+    upload(c, { { z, zl, dz.get(), zl } });
     const int m_pad = static_cast<int>(round_up(mt, 64));
     if (const ForwardSolve how = forward_solve(m, mt); how != ForwardSolve::Blocked)
     {
@@ -1645,7 +1739,7 @@ void predict_with_uncertainty_once(Context &c, const double *x, std::size_t x_le
     require(z != nullptr && z_len >= static_cast<std::size_t>(mt) + r - 1, "predict: test input must hold m + n_reg - 1 values");
     require(theta != nullptr && mean != nullptr && var != nullptr, "predict: null argument");
     require(y != nullptr && y_len >= static_cast<std::size_t>(n), "training output must hold n values");
-    c.make_current();
+    c.begin_call();
     Model m;
     m.ctx = &c;
     m.n = n;
@@ -1662,35 +1756,30 @@ void predict_with_uncertainty_once(Context &c, const double *x, std::size_t x_le
     m.L = DevBuf<double>(c, (static_cast<std::size_t>(m.n_pad) + extra) * m.lda);
     m.Winv = DevBuf<double>(c, static_cast<std::size_t>(m.n_pad) * 64);
     DevBuf<double> dz(c, zl);
-    upload(c, m.x.get(), x, xl);
-    upload(c, dz.get(), z, zl);
     double *rows = m.L.get() + static_cast<long>(m.n_pad) * m.lda;
     double *yrow = rows + static_cast<long>(m_pad) * m.lda;
+    // (of the last block only the targets' row is read again)
+    upload(c, { { x, xl, m.x.get(), xl }, { z, zl, dz.get(), zl }, { y, static_cast<std::size_t>(n), yrow, static_cast<std::size_t>(m.n_pad) } });
     {
         Timed t(c, c.main, "assemble");
         k::assemble_lower(c.main, m.x.get(), r, m.sek, m.L.get(), m.lda, n, m.n_pad);
         k::assemble_cross_rows(c.main, m.x.get(), dz.get(), r, m.sek, rows, m.lda, n, m.n_pad, mt, m_pad);
-        k::fill(c.main, yrow, 64L * m.lda, 0.0);
-        GP_HIP(hipMemcpyAsync(yrow, y, sizeof(double) * n, hipMemcpyDefault, c.main));
     }
     // the rows below K come out as K* L^-T (test row t: v_t = L^-1 k_t) and
     // (L^-1 y)^T, so the mean is K* K^-1 y = V (L^-1 y) and the variance
     // v - |v_t|^2: no alpha and no separate solve
     cholesky(c, m.L.get(), m.lda, m.n_pad, m.Winv.get(), false, nullptr, extra);
-    DevBuf<double> dmean(c, mt), colsq(c, mt), dvar(c, mt);
+    Result means(c, mean, mt), vars(c, var, mt);
     {
         Timed t(c, c.main, "mean");
-        k::rowdot(c.main, rows, m.lda, m.n_pad, mt, yrow, dmean.get(), false);
+        k::rows_mean_variance(c.main, rows, m.lda, mt, m.n_pad, yrow, m.sek.vertical, means.get(), vars.get());
     }
-    {
-        Timed t(c, c.main, "variance_rows");
-        k::row_sumsq(c.main, rows, m.lda, mt, m.n_pad, colsq.get());
-        k::variance_finish(c.main, colsq.get(), m.sek.vertical, mt, dvar.get());
-    }
-    GP_HIP(hipMemcpyAsync(mean, dmean.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
-    GP_HIP(hipMemcpyAsync(var, dvar.get(), sizeof(double) * mt, hipMemcpyDefault, c.main));
+    means.send();
+    vars.send();
     c.sync();
     check_pivots(c);
+    means.deliver();
+    vars.deliver();
 }
 
 FactorView view(const Model &m)
@@ -1820,12 +1909,11 @@ static double loss_of(const Model &m, const double *t);
 double loss(Model &m)
 {
     Context &c = *m.ctx;
-    c.make_current();
-    k::loss_terms(c.main, m.L.get(), m.lda, m.y.get(), m.alpha.get(), m.n, c.scalars.get());
-    double t[3];
-    GP_HIP(hipMemcpyAsync(t, c.scalars.get(), sizeof t, hipMemcpyDefault, c.main));
+    c.begin_call();
+    Result t(c, nullptr, 3);
+    k::loss_terms(c.main, m.L.get(), m.lda, m.y.get(), m.alpha.get(), m.n, t.get());
     c.sync();
-    return loss_of(m, t);
+    return loss_of(m, t.get());
 }
 
 // Softplus chain factors, as core/src/cpu/gp_optimizer.cpp:12-36.
@@ -1915,16 +2003,15 @@ void loss_gradient(Context &c,
     // a row of targets as z = L^-1 y; then alpha = W^T z
     require(y != nullptr && y_len >= static_cast<std::size_t>(n), "training output must hold n values");
     check_training(x, x_len, n, r, theta, GPRAT_PRECISION_FP64);
-    c.make_current();
+    c.begin_call();
+    double *h = c.stage_take(64);  // the scalar results; first, so that it fits
     const int extra = n_pad + 64;
     const bool flow = one_launch(n_pad, false, extra, n_pad);
     const long lda = leading_dim(n_pad);
     DevBuf<double> X;
     m.y = DevBuf<double>(c, n_pad);
-    k::fill(c.main, m.y.get(), n_pad, 0.0);
-    upload(c, m.y.get(), y, static_cast<std::size_t>(n));
     double *z = nullptr, *WT = nullptr;
-    auto targets = [&] { GP_HIP(hipMemcpyAsync(z, m.y.get(), sizeof(double) * n_pad, hipMemcpyDeviceToDevice, c.main)); };
+    auto targets = [&] { upload(c, { { y, static_cast<std::size_t>(n), m.y.get(), static_cast<std::size_t>(n_pad), z } }); };
     Riding riding;
     riding.extra = extra;
     riding.unit = n_pad;
@@ -1977,8 +2064,7 @@ void loss_gradient(Context &c,
         Timed t(c, c.main, "gradient");
         k::gradient_sums(c.main, m.L.get(), lda, m.x.get(), m.alpha.get(), r, m.sek, sig_l, sig_v, n, part.get(), c.scalars.get() + 8);
     }
-    double h[13];
-    GP_HIP(hipMemcpyAsync(h, c.scalars.get(), sizeof h, hipMemcpyDefault, c.main));
+    k::report(c.main, c.scalars.get(), 64, h, c.info.get(), c.host_info);
     c.sync();
     check_pivots(c);
     gradient_results(m, h, h + 8, trainable, loss_out, grad);

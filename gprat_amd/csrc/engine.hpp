@@ -129,6 +129,15 @@ struct Context
 
     DevBuf<int> info;         // smallest non-positive pivot column
     int *host_info = nullptr; // its pinned copy (check_pivots)
+    // Pinned staging of a call's small inputs and results, which kernels read
+    // and write in place (a copy from or to pageable memory costs the host 8
+    // to 25 us each): taken front to back, all free again at begin_call().
+    static constexpr std::size_t STAGE = std::size_t(1) << 17;  // doubles
+    double *stage = nullptr;
+    std::size_t stage_used = 0;
+    bool stage_busy = false;  // taken from since the last sync()
+    void begin_call();
+    double *stage_take(std::size_t count);  // null if it does not fit
     DevBuf<double> scalars;   // reduction results
 
     // profiling

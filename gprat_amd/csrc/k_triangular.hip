@@ -857,6 +857,66 @@ __global__ void k_to_f32(const double *__restrict__ src, float *__restrict__ dst
         dst[i] = static_cast<float>(src[i]);
 }
 
+struct PlaceItems
+{
+    PlaceItem item[3];
+};
+
+__global__ __launch_bounds__(THREADS) void k_place(PlaceItems p)
+{
+    const PlaceItem &t = p.item[blockIdx.y];
+    const int i = blockIdx.x * THREADS + threadIdx.x;
+    if (i >= t.n_pad)
+        return;
+    const double v = i < t.n ? t.src[i] : 0.0;
+    t.dst[i] = v;
+    if (t.also)
+        t.also[i] = v;
+}
+
+__global__ void k_report(const double *__restrict__ values, int count, double *__restrict__ out, const int *__restrict__ info, int *__restrict__ out_info)
+{
+    if (static_cast<int>(threadIdx.x) < count)
+        out[threadIdx.x] = values[threadIdx.x];
+    if (threadIdx.x == 0)
+        *out_info = *info;
+}
+
+// One workgroup per row: both sums in one pass over it.
+__global__ __launch_bounds__(THREADS) void k_rows_mean_variance(const double *__restrict__ S, long lds, int cols, const double *__restrict__ z, double v,
+                                                                double *__restrict__ dot, double *__restrict__ var)
+{
+    __shared__ double red[2][THREADS];
+    const double *row = S + static_cast<long>(blockIdx.x) * lds;
+    const int tid = threadIdx.x;
+    double s = 0.0, q = 0.0;
+    for (int i = 2 * tid; i < cols; i += 2 * THREADS)
+    {
+        const blk::d2 a = *reinterpret_cast<const blk::d2 *>(row + i), b = *reinterpret_cast<const blk::d2 *>(z + i);
+        s = fma(a[0], b[0], s);
+        q = fma(a[0], a[0], q);
+        s = fma(a[1], b[1], s);
+        q = fma(a[1], a[1], q);
+    }
+    red[0][tid] = s;
+    red[1][tid] = q;
+    __syncthreads();
+    for (int h = THREADS / 2; h > 0; h >>= 1)
+    {
+        if (tid < h)
+        {
+            red[0][tid] += red[0][tid + h];
+            red[1][tid] += red[1][tid + h];
+        }
+        __syncthreads();
+    }
+    if (tid == 0)
+    {
+        dot[blockIdx.x] = red[0][0];
+        var[blockIdx.x] = v - red[1][0];
+    }
+}
+
 }  // namespace
 
 void invert_blocks256(hipStream_t s, const double *L, long lda, const double *Winv, long row0, long rows, double *Wt, long ldw,
@@ -1054,6 +1114,36 @@ void add_vec(hipStream_t s, double *y, const double *x, long n)
     if (n <= 0)
         return;
     hipLaunchKernelGGL(k_add_vec, dim3(ceil_div(n, 256)), dim3(256), 0, s, y, x, n);
+    GP_CHECK_LAUNCH();
+}
+
+void place(hipStream_t s, const PlaceItem *items, int count)
+{
+    require(count >= 1 && count <= 3, "place: 1 to 3 items");
+    PlaceItems p{};
+    int most = 1;
+    for (int i = 0; i < count; i++)
+    {
+        require(items[i].n >= 0 && items[i].n_pad >= items[i].n, "place: bad item");
+        p.item[i] = items[i];
+        most = std::max(most, items[i].n_pad);
+    }
+    hipLaunchKernelGGL(k_place, dim3(static_cast<unsigned>(ceil_div(most, THREADS)), count), dim3(THREADS), 0, s, p);
+    GP_CHECK_LAUNCH();
+}
+
+void report(hipStream_t s, const double *values, int count, double *out, const int *info, int *out_info)
+{
+    require(count >= 0 && count <= 64, "report: at most 64 values");
+    hipLaunchKernelGGL(k_report, dim3(1), dim3(64), 0, s, values, count, out, info, out_info);
+    GP_CHECK_LAUNCH();
+}
+
+void rows_mean_variance(hipStream_t s, const double *S, long lds, int rows, int cols, const double *z, double v, double *dot, double *var)
+{
+    require(rows >= 1 && cols >= 2 && cols % 2 == 0 && lds % 2 == 0 && lds >= cols, "rows_mean_variance: bad shape");
+    require(reinterpret_cast<uintptr_t>(S) % 16 == 0 && reinterpret_cast<uintptr_t>(z) % 16 == 0, "rows_mean_variance: operands must be 16-byte aligned");
+    hipLaunchKernelGGL(k_rows_mean_variance, dim3(static_cast<unsigned>(rows)), dim3(THREADS), 0, s, S, lds, cols, z, v, dot, var);
     GP_CHECK_LAUNCH();
 }
 

@@ -337,6 +337,24 @@ void subtract_row_products(hipStream_t s, const double *V, long ldv, int n, doub
 // out[i * n + j] = S[i * lds + j] for i, j < n.
 void pack_square(hipStream_t s, const double *S, long lds, int n, double *out);
 
+// ---- host staging (k_triangular.hip) --------------------------------------
+
+// dst[i] (and also[i], if given) = src[i] for i < n, 0 for n <= i < n_pad, for
+// `count` (1 .. 3) items in one launch; src may be pinned host memory.
+struct PlaceItem
+{
+    const double *src;
+    double *dst, *also;
+    int n, n_pad;
+};
+void place(hipStream_t s, const PlaceItem *items, int count);
+// out[i] = values[i] for i < count, *out_info = *info: out and out_info may be
+// pinned host memory (count may be 0).
+void report(hipStream_t s, const double *values, int count, double *out, const int *info, int *out_info);
+// Per row j < rows of S (row stride lds, cols values): dot[j] = row . z and
+// var[j] = v - |row|^2, in a fixed order; outputs may be pinned host memory.
+void rows_mean_variance(hipStream_t s, const double *S, long lds, int rows, int cols, const double *z, double v, double *dot, double *var);
+
 // ---- few right-hand sides (k_few.hip) -------------------------------------
 
 // V = X L^-T for `rows` (a multiple of 16) rows X of n values, stepping

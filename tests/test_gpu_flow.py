@@ -119,3 +119,21 @@ def test_forward_solves_agree(ctx, n, m):
         assert norm_rel(out[how][1], out["2"][1]) < TOL
         assert norm_rel(out[how][2].ravel(), out["2"][2].ravel()) < TOL
         assert np.array_equal(out[how][2], out[how][2].T)
+
+
+@pytest.mark.parametrize("n", [200, 1100])
+def test_device_memory_in_and_out(ctx, n):
+    """Results through pinned staging (host arrays) and through device buffers are the same."""
+    m, theta = 77, (1.0, 1.0, 0.1)
+    x, y, z = datagen.gp_problem(n, m, 8)
+    dx, dy, dz = (ctx.device_array(v) for v in (x, y, z))
+    out = ctx.device_empty(m), ctx.device_empty(m)
+    host = ctx.predict(x, y, z, theta, 1, n, 1, m, 8, variance=True)
+    ctx.predict(dx, dy, dz, theta, 1, n, 1, m, 8, variance=True, out=out)
+    assert all(np.array_equal(h, d.numpy()) for h, d in zip(host, out))
+    a, b = ctx.fit(x, y, n, 8, theta), ctx.fit(dx, dy, n, 8, theta)
+    b.predict(dz, m, out=out)
+    assert a.loss() == b.loss()
+    assert all(np.array_equal(h, d.numpy()) for h, d in zip(a.predict(z, m), out))
+    a.release()
+    b.release()
