@@ -672,6 +672,23 @@ __global__ __launch_bounds__(THREADS) void k_pack_square(const double *__restric
 
 long flow_counters(int nb, int ne) { return 1 + (static_cast<long>(nb) + ne) * (1 + nb); }
 
+// Workgroups of a launch: enough for the work to keep up with the chain
+// (products of 64x64 blocks, 4 us each with two workgroups on a CU, over 15 us
+// per block column, 8 on a given factor), and some that wait ahead; more only
+// share the chain's CU and poll. Two workgroups' LDS fit a CU. Measured on
+// MI355X (one call, 128 / 192 / 256 / 384 / 512 workgroups, us):
+//   n = 1024 m = 1024 330 351 363 379 393     n = 2048 m = 1024 733 704 730 808 860
+//   n = 3000 m = 64 - 1006 1005 1072 1147     n = 4096 m = 16 1797 1584 1523 1622 1723
+//   n = 6144 m = 16 - 3757 3380 3173 3177     n = 8192 m = 16 - 8291 7085 6252 6056
+static long flow_workgroups(const FlowCall &f, int cus)
+{
+    const double nb = f.nb, ne = f.ne - f.nu, nu = f.nu;
+    const double rows = (f.solve ? 0.0 : nb / 6) + ne / 2 + nu / 6;  // products per column and block row of columns
+    const double need = rows * nb * (f.solve ? 4.0 / 8 : 4.0 / 15);
+    const long wgs = static_cast<long>((need + 80) / 64 + 0.5) * 64;
+    return std::clamp<long>(wgs, std::min(cus / 2, 128), 2L * cus);
+}
+
 void flow_cholesky(hipStream_t s, const FlowCall &f, int cus)
 {
     require(f.nb >= 1 && f.ne >= 0 && f.lda % 2 == 0 && f.lda >= static_cast<long>(NB) * f.nb, "flow_cholesky: bad shape");
@@ -695,7 +712,7 @@ void flow_cholesky(hipStream_t s, const FlowCall &f, int cus)
     a.tasks = static_cast<int>(tasks);
     hipLaunchKernelGGL(k_flow_init, dim3(static_cast<unsigned>(ceil_div(counters, THREADS))), dim3(THREADS), 0, s, a, counters);
     GP_CHECK_LAUNCH();
-    const long wgs = std::min<long>(tasks, 2L * cus);  // two workgroups' LDS fit a CU
+    const long wgs = std::min<long>(tasks, flow_workgroups(f, cus));
     if (f.solve)
         hipLaunchKernelGGL(k_flow<true>, dim3(static_cast<unsigned>(wgs)), dim3(THREADS), 0, s, a);
     else
