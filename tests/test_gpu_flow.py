@@ -80,6 +80,16 @@ def test_tiles(ctx, n):
     assert norm_rel(a.ravel(), b.ravel()) < TOL
 
 
+@pytest.mark.parametrize("n", SIZES)
+def test_gradient(ctx, n):
+    x, y, _ = datagen.gp_problem(n, 1, 8)
+    theta = (1.0, 1.0, 0.1)
+    loss, grad = ctx.loss_gradient(x, y, theta, 1, n, 8)
+    with panel_schedule():
+        ploss, pgrad = ctx.loss_gradient(x, y, theta, 1, n, 8)
+    assert norm_rel(np.atleast_1d(loss), np.atleast_1d(ploss)) < TOL and norm_rel(grad, pgrad) < 10 * TOL
+
+
 def test_repeats_are_bit_identical(ctx):
     x, y, z = datagen.gp_problem(1800, 300, 8)
     args = (x, y, z, (1.0, 1.0, 0.1), 1, 1800, 1, 300, 8)
