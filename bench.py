@@ -708,13 +708,13 @@ def main():
     n_pad = ((HN + 127) // 128) * 128
     m_pad = ((HM + 63) // 64) * 64
     trailing = trailing_update_flops(n_pad)
-    r_fp32 = roofline_of("k_gemm_f32_tn<double,0> (FP32 matrix-core trailing update of the mixed-precision Cholesky)",
+    r_fp32 = roofline_of("k_gemm_f32_tn<double> (FP32 matrix-core trailing update of the mixed-precision Cholesky)",
                          sum(trailing) / len(trailing), fams["syrk_trailing"], FP32_MFMA_PEAK_TFLOPS,
                          "trailing_update_f32_n32768_traffic.md")
     r_res = roofline_of("k_gemm_f64<true,false,8> (FP64 residual product K_sl X of the variance refinement)",
                         residual_flops(n_pad, m_pad), fams["residual"], FP64_MFMA_PEAK_TFLOPS, "residual_n32768_traffic.md")
     upd_flops, upd_launches = variance_update_flops(n_pad, m_pad, outer_block(n_pad), 2)
-    r_upd = roofline_of("k_gemm_f32_tn<float,2> (FP32 matrix-core updates of the variance's forward and backward solves)",
+    r_upd = roofline_of("k_gemm_f32_solve (FP32 matrix-core updates of the variance's forward and backward solves)",
                         upd_flops / upd_launches, fams["trsm_update"], FP32_MFMA_PEAK_TFLOPS, "trsm_update_f32_n32768_traffic.md")
     ranked = sorted([r for r in (r_fp32, r_res, r_upd) if r], key=lambda r: -r["launches"] * r["avg_launch_ms"])
     roofline = ranked[0] if ranked else None

@@ -902,7 +902,7 @@ struct VarianceF32
     using T = float;
     static void leaf(hipStream_t s, const T *W, int ldw, const T *B, long ldb, T *V, int nb, int cols)
     {
-        k::gemm_f32_tn(s, W, ldw, B, ldb, V, ldb, nb, cols, nb, true, 0, true);  // W_J lower triangular
+        k::gemm_f32_tn(s, W, ldw, B, ldb, V, ldb, nb, cols, nb, true, k::Triangle::Lower);
     }
     static void update(hipStream_t s, const T *P, long ldp, const T *V, long ldv, T *B, long ldb, int M, int cols, int K)
     {
@@ -1060,7 +1060,7 @@ static void backward_solve_f32(Context &c, const double *L, long lda, const floa
         const int j0 = J * NBK, nb = std::min(NBK, n_pad - j0);
         hipEvent_t next = J - 1 >= 1 ? copy(J - 1) : nullptr;
         float *BJ = B + static_cast<long>(j0) * m_pad;
-        k::gemm_f32_tn(s, WT + static_cast<long>(J) * NBK * NBK, NBK, BJ, m_pad, T.get(), m_pad, nb, m_pad, nb, true);
+        k::gemm_f32_tn(s, WT + static_cast<long>(J) * NBK * NBK, NBK, BJ, m_pad, T.get(), m_pad, nb, m_pad, nb, true, k::Triangle::Upper);
         GP_HIP(hipMemcpyAsync(BJ, T.get(), sizeof(float) * nb * m_pad, hipMemcpyDeviceToDevice, s));
         if (j0 == 0)
             break;

@@ -4,12 +4,13 @@
 // The factored FP64 panel is first copied to FP32 in k-major order
 // (P[k][row], `panel_to_f32t`), so both operands of C -= A B^T are read as
 // contiguous 16-byte row segments and land in LDS without a transpose.
-// One workgroup (4 wavefronts) owns a 128x128 tile of the FP64 trailing
-// matrix; each wavefront accumulates a 64x64 quarter in FP32 on
+// One workgroup (4 wavefronts) owns a 128x128 tile (short solve products:
+// 64x64); each wavefront accumulates a quarter in FP32 on
 // v_mfma_f32_16x16x4f32 over 16-deep LDS slabs (double buffered), and the
 // epilogue subtracts the FP32 product from the FP64 matrix. The shallow
-// slabs (36 KiB of LDS per workgroup) and a 168-register budget let a CU
-// hold three workgroups; on MI355X that ran the variance solve's updates at
+// slabs (36 KiB of LDS per workgroup; 40 KiB for the small tile, whose
+// slabs are 32 deep so that a load's latency is paid half as often) and a
+// 168-register budget let a CU hold three workgroups; on MI355X that ran the variance solve's updates at
 // 124 TF/s against 118 with 32-deep slabs and two workgroups.
 #include "kernels.hpp"
 
@@ -23,11 +24,22 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // stay in registers (the HIP float4 struct ends up in scratch here)
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-constexpr int BM = 128;
-constexpr int BK = 16;
-constexpr int LPT = BK * 128 / (256 * 4);  // 16-byte loads per thread per operand slab
-constexpr int KS = BM + 16;  // floats per LDS k-row: the 4 k-slots of a read hit disjoint banks
 constexpr int THREADS = 256;
+
+// Tile shapes: B x B elements of C per workgroup, one quarter per wavefront,
+// over D-deep slabs. The sums run in the same k order in both, so an element
+// does not depend on the shape that computed it.
+template <int B, int D>
+struct Tile
+{
+    static constexpr int BM = B, BK = D;
+    static constexpr int Q = B / 2, NI = B / 32;        // a wavefront's quarter, in elements and 16-wide blocks
+    static constexpr int LPT = D * B / (THREADS * 4);  // 16-byte loads per thread per operand slab
+    static constexpr int KS = B + 16;  // floats per LDS k-row: the 4 k-slots of a read hit disjoint banks
+};
+using Large = Tile<128, 16>;
+using Small = Tile<64, 32>;
+constexpr int BM = Large::BM;
 
 // C (op)= A B with A(i, k) = A[k * lda + i] and B(k, j) = B[k * ldb + j]
 // (both operands k-major, as the panel copies are), FP32 products and sums.
@@ -46,6 +58,7 @@ struct Params32
     int set;  // C = acc instead of C -= acc
     int max_wgs;  // > 0: at most this many workgroups, looping over tiles
     int k_to_row;  // A(i, k) known zero for k > i: each row tile stops K at its last row
+    int k_from_row;  // A(i, k) known zero for k < i: each row tile starts K at its first row
     int *queue;    // capped: tile counter (0 at launch) or null for fixed shares
     int tiles;     // capped: tiles holding part of the update
 };
@@ -53,73 +66,74 @@ struct Params32
 // Element offsets (within one slab) of this thread's LPT 16-byte loads,
 // clamped to the operand's last group of four; rows past the edge only feed
 // accumulators the epilogue never stores.
-__device__ __forceinline__ void slab_offsets(long ld, int rows, int tid, unsigned (&off)[LPT], int (&lds)[LPT])
+template <class S>
+__device__ __forceinline__ void slab_offsets(long ld, int rows, int tid, unsigned (&off)[S::LPT], int (&lds)[S::LPT])
 {
 #pragma unroll
-    for (int s = 0; s < LPT; s++)
+    for (int s = 0; s < S::LPT; s++)
     {
         const int idx = tid + THREADS * s;
-        const int kk = idx >> 5;         // 0..BK-1
-        const int col = (idx & 31) * 4;  // 0..124
+        const int kk = idx / (S::BM / 4);         // 0..BK-1
+        const int col = (idx % (S::BM / 4)) * 4;  // 0..BM-4
         off[s] = static_cast<unsigned>(kk * ld + min(col, rows - 4));
-        lds[s] = kk * KS + col;
+        lds[s] = kk * S::KS + col;
     }
 }
 
-__device__ __forceinline__ void mfma_slab32(const float *As, const float *Bs, int wr, int wc, int lm, int lk, v4f (&acc)[4][4])
+template <class S>
+__device__ __forceinline__ void mfma_slab32(const float *As, const float *Bs, int wr, int wc, int lm, int lk, v4f (&acc)[S::NI][S::NI])
 {
 #pragma unroll
-    for (int kq = 0; kq < BK / 4; kq++)
+    for (int kq = 0; kq < S::BK / 4; kq++)
     {
-        float a[4], b[4];
+        float a[S::NI], b[S::NI];
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-            a[i] = As[(kq * 4 + lk) * KS + wr * 64 + i * 16 + lm];
+        for (int i = 0; i < S::NI; i++)
+            a[i] = As[(kq * 4 + lk) * S::KS + wr * S::Q + i * 16 + lm];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            b[j] = Bs[(kq * 4 + lk) * KS + wc * 64 + j * 16 + lm];
+        for (int j = 0; j < S::NI; j++)
+            b[j] = Bs[(kq * 4 + lk) * S::KS + wc * S::Q + j * 16 + lm];
 #pragma unroll
-        for (int i = 0; i < 4; i++)
+        for (int i = 0; i < S::NI; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < S::NI; j++)
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
     }
 }
 
-// One 128x128 tile of C at (r0, c0).
-// C (op)= acc over one wavefront's 64x64 quarter, element (i, j, e) at
+// C (op)= acc over one wavefront's quarter of a tile, element (i, j, e) at
 // cw + (16 i + e) ldc + 16 j. C is read and written through the same
 // pointer, so the compiler keeps every element's load, wait and store in
 // program order; the loads of a 16-row strip are therefore all issued before
 // its first store (one memory latency per strip, not sixteen). FULL: an
 // interior tile (no edge, wholly inside the lower band), no predicates.
-template <bool FULL, class TC>
-__device__ __forceinline__ void store_quarter32(const Params32<TC> &p, const v4f (&acc)[4][4], TC *cw, int rb, int cb, int rows_a, int rows_b,
+template <bool FULL, int NI, class TC>
+__device__ __forceinline__ void store_quarter32(const Params32<TC> &p, const v4f (&acc)[NI][NI], TC *cw, int rb, int cb, int rows_a, int rows_b,
                                                 long r0, long c0)
 {
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < NI; i++)
     {
-        bool ok[16];
+        bool ok[4 * NI];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < NI; j++)
 #pragma unroll
             for (int e = 0; e < 4; e++)
             {
                 const int rr = rb + i * 16 + e, cc = cb + j * 16;
                 ok[j * 4 + e] = FULL || ((rr < rows_a) & (cc < rows_b) & !(p.lower && r0 + rr + p.diag_off < c0 + cc));
             }
-        TC cv[16];
+        TC cv[4 * NI];
         if (!p.set)
         {
 #pragma unroll
-            for (int j = 0; j < 4; j++)
+            for (int j = 0; j < NI; j++)
 #pragma unroll
                 for (int e = 0; e < 4; e++)
                     cv[j * 4 + e] = ok[j * 4 + e] ? cw[static_cast<long>(i * 16 + e) * p.ldc + j * 16] : TC(0);
         }
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < NI; j++)
 #pragma unroll
             for (int e = 0; e < 4; e++)
                 if (ok[j * 4 + e])
@@ -128,11 +142,13 @@ __device__ __forceinline__ void store_quarter32(const Params32<TC> &p, const v4f
     }
 }
 
+// One tile of C at (r0, c0).
 // part 0: the tile's whole K range; parts 1 and 2: its first and second
 // half (in slabs), for C -= updates only.
-template <class TC>
-__device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long c0, float (*As)[BK * KS], float (*Bs)[BK * KS], int part = 0)
+template <class S, class TC>
+__device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long c0, float (*As)[S::BK * S::KS], float (*Bs)[S::BK * S::KS], int part = 0)
 {
+    constexpr int BM = S::BM, BK = S::BK, LPT = S::LPT, NI = S::NI;
     const int rows_a = static_cast<int>(min(static_cast<long>(BM), p.M - r0));
     const int rows_b = static_cast<int>(min(static_cast<long>(BM), p.N - c0));
 
@@ -141,20 +157,21 @@ __device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long
     const int wr = wave >> 1, wc = wave & 1;
     const int lm = lane & 15, lk = lane >> 4;
 
-    v4f acc[4][4];
+    v4f acc[NI][NI];
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int i = 0; i < NI; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++)
+        for (int j = 0; j < NI; j++)
             acc[i][j] = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
 
     unsigned oa[LPT], ob[LPT];
     int la[LPT], lb[LPT];
-    slab_offsets(p.lda, rows_a, tid, oa, la);
-    slab_offsets(p.ldb, rows_b, tid, ob, lb);
+    slab_offsets<S>(p.lda, rows_a, tid, oa, la);
+    slab_offsets<S>(p.ldb, rows_b, tid, ob, lb);
     const int kmax = p.k_to_row ? static_cast<int>(min(static_cast<long>(p.K), r0 + BM)) : p.K;
+    const int kmin = p.k_from_row ? static_cast<int>(min(static_cast<long>(kmax), r0)) : 0;
     const int half = (kmax / BK / 2) * BK;
-    const int k0 = part == 2 ? half : 0, k1 = part == 1 ? half : kmax;
+    const int k0 = part == 2 ? half : kmin, k1 = part == 1 ? half : kmax;
     const float *ak = p.A + r0 + static_cast<long>(k0) * p.lda;
     const float *bk = p.B + c0 + static_cast<long>(k0) * p.ldb;
     const long astep = BK * p.lda, bstep = BK * p.ldb;
@@ -190,7 +207,7 @@ __device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long
         }
         // the next slab's loads stay ahead of this slab's products
         __builtin_amdgcn_sched_barrier(0);
-        mfma_slab32(As[buf], Bs[buf], wr, wc, lm, lk, acc);
+        mfma_slab32<S>(As[buf], Bs[buf], wr, wc, lm, lk, acc);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int s = 0; s < LPT; s++)
@@ -201,28 +218,39 @@ __device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long
         __syncthreads();
         buf ^= 1;
     }
-    mfma_slab32(As[buf], Bs[buf], wr, wc, lm, lk, acc);
+    mfma_slab32<S>(As[buf], Bs[buf], wr, wc, lm, lk, acc);
     }
 
     // Accumulator layout of the 16x16x4 f32 MFMA on gfx950: lane holds
     // column (lane % 16) and rows 4 (lane / 16) + e, e = 0..3.
     const bool full = rows_a == BM && rows_b == BM && (!p.lower || r0 + p.diag_off >= c0 + BM - 1);
-    const int er = wr * 64 + lk * 4, ec = wc * 64 + lm;
+    const int er = wr * S::Q + lk * 4, ec = wc * S::Q + lm;
     TC *cw = p.C + (r0 + er) * p.ldc + c0 + ec;
     if (full)
-        store_quarter32<true>(p, acc, cw, er, ec, rows_a, rows_b, r0, c0);
+        store_quarter32<true, NI>(p, acc, cw, er, ec, rows_a, rows_b, r0, c0);
     else
-        store_quarter32<false>(p, acc, cw, er, ec, rows_a, rows_b, r0, c0);
+        store_quarter32<false, NI>(p, acc, cw, er, ec, rows_a, rows_b, r0, c0);
 }
 
-// ROLE only separates profiler names: 0 trailing update (FP64 C), 1 TRSM
-// diagonal step, 2 TRSM update. Tiles are numbered row-major; a launch with
-// fewer workgroups than tiles loops over them (tile w, w + G, ...).
-template <class TC, int ROLE>
+// The solves' products, one workgroup per tile, row-major. ROLE only
+// separates profiler names: 1 diagonal step, 2 update.
+template <class S, int ROLE>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_gemm_f32_solve(Params32<float> p)
+{
+    __shared__ float As[2][S::BK * S::KS];
+    __shared__ float Bs[2][S::BK * S::KS];
+    const unsigned gx = (p.N + S::BM - 1) / S::BM;
+    gemm_tile32<S, float>(p, static_cast<long>(blockIdx.x / gx) * S::BM, static_cast<long>(blockIdx.x % gx) * S::BM, As, Bs);
+}
+
+// The factorisation's trailing update (FP64 C). Tiles are numbered
+// row-major; a launch with fewer workgroups than tiles loops over them
+// (tile w, w + G, ...).
+template <class TC>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_gemm_f32_tn(Params32<TC> p)
 {
-    __shared__ float As[2][BK * KS];
-    __shared__ float Bs[2][BK * KS];
+    __shared__ float As[2][Large::BK * Large::KS];
+    __shared__ float Bs[2][Large::BK * Large::KS];
     const int gx = (p.N + BM - 1) / BM;
     const int gy = (p.M + BM - 1) / BM;
     if (p.max_wgs <= 0)
@@ -231,7 +259,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) vo
         const long r0 = static_cast<long>(blockIdx.x / gx) * BM, c0 = static_cast<long>(blockIdx.x % gx) * BM;
         if (p.lower && r0 + (BM - 1) + p.diag_off < c0)
             return;
-        gemm_tile32<TC>(p, r0, c0, As, Bs, 0);
+        gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 0);
         return;
     }
     // Capped: the tiles holding part of the update (for a lower update, those
@@ -256,18 +284,18 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) vo
     auto run = [&](int t, long r0, long c0)
     {
         if (p.set || t < G / 2 || t >= G)
-            gemm_tile32<TC>(p, r0, c0, As, Bs, 0);
+            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 0);
         else if (first_r < 0)
         {
             first_r = r0;
             first_c = c0;
-            gemm_tile32<TC>(p, r0, c0, As, Bs, 1);
+            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 1);
         }
         else
         {
-            gemm_tile32<TC>(p, r0, c0, As, Bs, 1);
+            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 1);
             __syncthreads();
-            gemm_tile32<TC>(p, r0, c0, As, Bs, 2);
+            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 2);
         }
     };
     if (p.queue)
@@ -309,7 +337,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) vo
     if (first_r >= 0)
     {
         __syncthreads();
-        gemm_tile32<TC>(p, first_r, first_c, As, Bs, 2);
+        gemm_tile32<Large, TC>(p, first_r, first_c, As, Bs, 2);
     }
 }
 
@@ -365,54 +393,82 @@ void panel_to_f64t(hipStream_t s, const double *A, long lda, long r0, long p0, i
     panel_to_t<double>(s, A, lda, r0, p0, R, W, P, ldp, back, ldback);
 }
 
-template <class TC, int ROLE>
-static void launch_f32_tn(hipStream_t s, const Params32<TC> &p)
+template <class TC>
+static void check_f32(const Params32<TC> &p)
 {
-    if (p.M <= 0 || p.N <= 0)
-        return;
-    require(p.K % BK == 0, "FP32 product: K must be a multiple of 16");
+    require(p.K % Large::BK == 0, "FP32 product: K must be a multiple of 16");
     require(p.M % 4 == 0 && p.N % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0
                 && reinterpret_cast<uintptr_t>(p.A) % 16 == 0 && reinterpret_cast<uintptr_t>(p.B) % 16 == 0,
             "FP32 product: operand rows must come in aligned groups of four");
-    require(static_cast<long>(BK) * std::max(p.lda, p.ldb) + BM < (1L << 31), "FP32 product: operand too tall");
-    const long gx = ceil_div(static_cast<long>(p.N), static_cast<long>(BM)), gy = ceil_div(static_cast<long>(p.M), static_cast<long>(BM));
-    require(gx * gy < (1L << 31), "FP32 product: too many tiles for one launch");
-    // tiles holding part of the update, counted as the capped kernel numbers them
-    long active = 0;
-    for (long tr = 0; tr < gy; tr++)
-    {
-        const long last = tr * BM + (BM - 1) + p.diag_off;
-        active += p.lower ? (last < 0 ? 0 : std::min(gx, last / BM + 1)) : gx;
-    }
-    if (active == 0)
-        return;
-    Params32<TC> q = p;
-    q.tiles = static_cast<int>(std::min(active, (1L << 30)));
-    if (q.max_wgs >= active)
-    {
-        q.max_wgs = 0;  // the cap does not bind: one workgroup per tile
-        q.queue = nullptr;
-    }
-    dim3 grid(static_cast<unsigned>(q.max_wgs > 0 ? q.max_wgs : gx * gy));
-    hipLaunchKernelGGL((k_gemm_f32_tn<TC, ROLE>), grid, dim3(THREADS), 0, s, q);
-    GP_CHECK_LAUNCH();
+    require(static_cast<long>(Small::BK) * std::max(p.lda, p.ldb) + BM < (1L << 31), "FP32 product: operand too tall");
 }
 
 void gemm_f32_trailing(hipStream_t s, const float *P, long ldp, long a_off, long b_off, double *C, long ldc, int M, int N, int K, long diag_off,
                        int max_wgs, int *queue)
 {
-    Params32<double> p{ P + a_off, ldp, P + b_off, ldp, C, ldc, M, N, K, 1, diag_off, 0, max_wgs, 0, queue, 0 };
-    launch_f32_tn<double, 0>(s, p);
+    if (M <= 0 || N <= 0)
+        return;
+    Params32<double> p{ P + a_off, ldp, P + b_off, ldp, C, ldc, M, N, K, 1, diag_off, 0, max_wgs, 0, 0, queue, 0 };
+    check_f32(p);
+    const long gx = ceil_div(static_cast<long>(N), static_cast<long>(BM)), gy = ceil_div(static_cast<long>(M), static_cast<long>(BM));
+    require(gx * gy < (1L << 31), "FP32 product: too many tiles for one launch");
+    // tiles holding part of the update, counted as the capped kernel numbers them
+    long active = 0;
+    for (long tr = 0; tr < gy; tr++)
+    {
+        const long last = tr * BM + (BM - 1) + diag_off;
+        active += last < 0 ? 0 : std::min(gx, last / BM + 1);
+    }
+    if (active == 0)
+        return;
+    p.tiles = static_cast<int>(std::min(active, (1L << 30)));
+    if (p.max_wgs >= active)
+    {
+        p.max_wgs = 0;  // the cap does not bind: one workgroup per tile
+        p.queue = nullptr;
+    }
+    dim3 grid(static_cast<unsigned>(p.max_wgs > 0 ? p.max_wgs : gx * gy));
+    hipLaunchKernelGGL(k_gemm_f32_tn<double>, grid, dim3(THREADS), 0, s, p);
+    GP_CHECK_LAUNCH();
+}
+
+// The solves' products take 64x64 tiles where 128x128 ones would number at
+// most this many. A diagonal step is 6 tile rows of 128 (72 tiles for 1536
+// columns: under a third of the CUs, each alone with its 2048 matrix cycles
+// per slab), and an update near the end of its sweep is as short; a quarter
+// tile per workgroup fills the CUs and evens out the last wave. Above it the
+// operands, read twice as often, cost more than the last wave does. Variance
+// requests on MI355X (128x128 tiles only / small up to 400 / 1000 /
+// 2000 / always): n = 12000, 300 columns 7.63 / 4.85 / 4.85 / 4.84 ms,
+// 1500 columns 11.55 / 10.03 / 9.85 / 9.84, 8192 columns 42.4 / 41.7 / 41.6 /
+// 41.7; n = 24000, 700 columns 22.95 / - / 18.58 / 18.24 / 18.26, 8192
+// columns 155.9 / - / 155.8 / 155.4 / 158.1. A diagonal step at 1536 columns
+// went from 53 to 18 us, a third of that from leaving out the half of W_J
+// that is zero.
+constexpr long SMALL_TILE_LIMIT = 2048;
+
+template <class S, int ROLE>
+static void launch_solve(hipStream_t s, const Params32<float> &p)
+{
+    const long tiles = ceil_div(static_cast<long>(p.N), static_cast<long>(S::BM)) * ceil_div(static_cast<long>(p.M), static_cast<long>(S::BM));
+    require(tiles < (1L << 31), "FP32 product: too many tiles for one launch");
+    hipLaunchKernelGGL((k_gemm_f32_solve<S, ROLE>), dim3(static_cast<unsigned>(tiles)), dim3(THREADS), 0, s, p);
+    GP_CHECK_LAUNCH();
 }
 
 void gemm_f32_tn(hipStream_t s, const float *A, long lda, const float *B, long ldb, float *C, long ldc, int M, int N, int K, bool set,
-                 int max_wgs, bool a_lower)
+                 Triangle a)
 {
-    Params32<float> p{ A, lda, B, ldb, C, ldc, M, N, K, 0, 0, set ? 1 : 0, max_wgs, a_lower ? 1 : 0, nullptr, 0 };
+    if (M <= 0 || N <= 0)
+        return;
+    Params32<float> p{ A, lda, B, ldb, C, ldc, M, N, K, 0, 0, set ? 1 : 0, 0, a == Triangle::Lower, a == Triangle::Upper, nullptr, 0 };
+    check_f32(p);
+    const long large = ceil_div(static_cast<long>(N), static_cast<long>(BM)) * ceil_div(static_cast<long>(M), static_cast<long>(BM));
+    const bool small = K % Small::BK == 0 && large <= SMALL_TILE_LIMIT;
     if (set)
-        launch_f32_tn<float, 1>(s, p);
+        small ? launch_solve<Small, 1>(s, p) : launch_solve<Large, 1>(s, p);
     else
-        launch_f32_tn<float, 2>(s, p);
+        small ? launch_solve<Small, 2>(s, p) : launch_solve<Large, 2>(s, p);
 }
 
 }  // namespace gpamd::k

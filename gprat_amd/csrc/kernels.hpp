@@ -166,9 +166,11 @@ void gemm_f32_trailing(hipStream_t s, const float *P, long ldp, long a_off, long
                        int max_wgs = 0, int *queue = nullptr);
 // C (= or -=) A B over FP32 operands, A(i,k) = A[k*lda + i], B(k,j) = B[k*ldb + j],
 // FP32 C; K % 16 == 0, M, N, lda, ldb multiples of 4, A and B 16-byte aligned.
-// a_lower: A(i, k) is known zero for k > i (each row tile stops K there)
+// A known triangular (Lower: zero for k > i, Upper: zero for k < i): each
+// row tile leaves out the K range where its A is zero.
+enum class Triangle { None, Lower, Upper };
 void gemm_f32_tn(hipStream_t s, const float *A, long lda, const float *B, long ldb, float *C, long ldc, int M, int N, int K, bool set,
-                 int max_wgs = 0, bool a_lower = false);
+                 Triangle a = Triangle::None);
 
 // ---- batched fit of many GPs (k_batch.hip) --------------------------------
 

@@ -147,3 +147,22 @@ def test_refined_variance_of_a_mixed_batch(ctx, oracle):
     om, ov = go.predict_with_uncertainty(list(z), mt, mb)
     print(f"mixed batch GP n={T * b}: mean {norm_rel(mean, om):.2e} var {norm_rel(var, ov):.2e}")
     assert norm_rel(mean, om) < MEAN and norm_rel(var, ov) < VAR
+
+
+@pytest.mark.parametrize("m", [1, 65, 300, 1500, 5000])
+def test_solve_tiles_agree(ctx, m, monkeypatch):
+    """The FP32 solves on 64x64 tiles (few columns) against 128x128 ones (the
+    first updates of 16000 columns): one column's FP32 sums run in the same
+    order in both, so the variances differ only by the FP64 reductions, whose
+    splits follow the column count: sqrt(5003) eps times terms of at most 1e4."""
+    from gprat_amd import capi, datagen
+    monkeypatch.setenv("GPRAT_FLOW_LIMIT", "0")  # a small model with a mixed factor
+    n = 5003
+    x, y, z = datagen.gp_problem(n, 16000, 8)
+    model = ctx.fit(x, y, n, 8, (1.0, 1.0, 0.1), capi.PRECISION_MIXED)
+    try:
+        var = model.predict(z, m)[1]
+        wide = model.predict(z, 16000)[1]
+    finally:
+        model.release()
+    assert norm_rel(var, wide[:m]) < 1e-10
