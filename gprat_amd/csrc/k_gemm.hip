@@ -3,11 +3,11 @@
 // One workgroup = 256 threads = 4 wavefronts computes a 128x128 tile of
 // C (op)= A * B; each wavefront owns a 64x64 quarter as a 4x4 grid of 16x16
 // MFMA accumulators (64 doubles per lane). K advances in chunks of 16
-// through a double-buffered LDS stage stored k-major ([k][row]), so each MFMA
-// operand is one ds_read_b64 per lane: lanes 0-15 read 16 consecutive rows
-// of k-slot 0, lanes 16-31 of k-slot 1, and so on. The LDS row stride of 144
-// doubles puts the four k-slots of a read in disjoint bank halves. The
-// steady-state loop has no branch and no predicated load, so the
+// through a double-buffered LDS stage stored k-major ([k][row]) and filled
+// from memory directly (gemm_tile.hpp), so each MFMA operand is one
+// ds_read_b64 per lane: lanes 0-15 read 16 consecutive rows of k-slot 0,
+// lanes 16-31 of k-slot 1, and so on. The LDS row stride of 144 doubles puts
+// the four k-slots of a read in disjoint bank halves. The steady-state loop has no branch and no predicated load, so the
 // accumulators stay in place and two workgroups share a CU.
 //
 // The same kernel serves the Cholesky trailing update (both operands the
@@ -32,8 +32,8 @@ using namespace gt;
 template <bool AT, bool BT, int ROLE>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64(Params p)
 {
-    __shared__ double As[2][BK * LDS_STRIDE];
-    __shared__ double Bs[2][BK * LDS_STRIDE];
+    __shared__ alignas(16) double As[2][BK * LDS_STRIDE];
+    __shared__ alignas(16) double Bs[2][BK * LDS_STRIDE];
     long r0 = static_cast<long>(blockIdx.y) * BM;
     const long c0 = static_cast<long>(blockIdx.x) * BN;
     if (p.k_before_tile)
@@ -80,8 +80,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
 template <bool AT, bool BT, int ROLE>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_gemm_f64_capped(Params p)
 {
-    __shared__ double As[2][BK * LDS_STRIDE];
-    __shared__ double Bs[2][BK * LDS_STRIDE];
+    __shared__ alignas(16) double As[2][BK * LDS_STRIDE];
+    __shared__ alignas(16) double Bs[2][BK * LDS_STRIDE];
     __shared__ int next;
     const int gx = (p.N + BN - 1) / BN;
     const int gy = (p.M + BM - 1) / BM;
@@ -95,65 +95,51 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(2, 2)))
         const long last = static_cast<long>(tr) * BM + (BM - 1) + p.diag_off;  // last column the band reaches
         return last < 0 ? 0 : static_cast<int>(min(static_cast<long>(gx), last / BN + 1));
     };
-    auto run = [&](int t, long r0, long c0)
+    // one loop, one copy of the tile's code: with a copy for each way to take
+    // a tile the kernel spilled 111 registers (26 with the direct LDS copies)
+    int tr = 0, row_first = 0, nc = gy > 0 ? row_tiles(0) : 0;  // the current tile row; tile numbers only grow
+    for (int t = blockIdx.x;; t += G)
     {
-        if (p.set || t < G / 2 || t >= G)
-            gemm_tile<AT, BT>(p, r0, c0, As, Bs, 0);
-        else if (first_r < 0)
+        if (p.queue)
         {
-            first_r = r0;
-            first_c = c0;
-            gemm_tile<AT, BT>(p, r0, c0, As, Bs, 1);
-        }
-        else
-        {
-            // a second split tile for this workgroup: both halves now
-            gemm_tile<AT, BT>(p, r0, c0, As, Bs, 1);
-            __syncthreads();
-            gemm_tile<AT, BT>(p, r0, c0, As, Bs, 2);
-        }
-    };
-    if (p.queue)
-    {
-        // tile numbers only grow, so the row walk is incremental
-        int tr = 0, row_first = 0, nc = gy > 0 ? row_tiles(0) : 0;
-        for (;;)
-        {
-            __syncthreads();  // the previous tile's LDS reads and `next` reads are done
+            __syncthreads();  // the previous tile's `next` reads are done
             if (threadIdx.x == 0)
                 next = atomicAdd(p.queue, 1);
             __syncthreads();
-            const int t = next;
-            if (t >= p.tiles)
-                break;
+            t = __builtin_amdgcn_readfirstlane(next);  // the tile's addresses stay in scalar registers
+        }
+        const bool done = t >= p.tiles;
+        if (done && first_r < 0)
+            break;
+        long r0 = first_r, c0 = first_c;
+        int part = 2, last = 2;  // with no other tile left: the deferred half
+        if (!done)
+        {
             while (t >= row_first + nc && tr + 1 < gy)
             {
                 row_first += nc;
                 nc = row_tiles(++tr);
             }
-            run(t, static_cast<long>(tr) * BM, static_cast<long>(t - row_first) * BN);
-        }
-    }
-    else
-    {
-        int rem = blockIdx.x;  // this workgroup's next tile, counted from the current row's first
-        int row_first = 0;     // number of the current row's first tile
-        for (int tr = 0; tr < gy; tr++)
-        {
-            const int nc = row_tiles(tr);
-            for (; rem < nc; rem += G)
+            r0 = static_cast<long>(tr) * BM;
+            c0 = static_cast<long>(t - row_first) * BN;
+            const bool whole = p.set || t < G / 2 || t >= G;
+            part = whole ? 0 : 1;
+            last = part;
+            if (!whole && first_r >= 0)
+                last = 2;  // a second split tile for this workgroup: both halves now
+            else if (!whole)
             {
-                __syncthreads();  // the previous tile's last slab has been read by every wavefront
-                run(row_first + rem, static_cast<long>(tr) * BM, static_cast<long>(rem) * BN);
+                first_r = r0;
+                first_c = c0;
             }
-            rem -= nc;
-            row_first += nc;
         }
-    }
-    if (first_r >= 0)
-    {
-        __syncthreads();
-        gemm_tile<AT, BT>(p, first_r, first_c, As, Bs, 2);
+        for (; part <= last; part++)
+        {
+            __syncthreads();  // the previous tile's last slab has been read by every wavefront
+            gemm_tile<AT, BT>(p, r0, c0, As, Bs, part);
+        }
+        if (done)
+            break;
     }
 }
 
