@@ -7,11 +7,15 @@
 // One workgroup (4 wavefronts) owns a 128x128 tile (short solve products:
 // 64x64); each wavefront accumulates a quarter in FP32 on
 // v_mfma_f32_16x16x4f32 over 16-deep LDS slabs (double buffered), and the
-// epilogue subtracts the FP32 product from the FP64 matrix. The shallow
-// slabs (36 KiB of LDS per workgroup; 40 KiB for the small tile, whose
-// slabs are 32 deep so that a load's latency is paid half as often) and a
-// 168-register budget let a CU hold three workgroups; on MI355X that ran the variance solve's updates at
-// 124 TF/s against 118 with 32-deep slabs and two workgroups.
+// epilogue subtracts the FP32 product from the FP64 matrix. The slabs go from
+// memory straight into LDS; they are shallow (32 KiB of LDS per workgroup,
+// also for the small tile, whose slabs are 32 deep so that a copy's latency is
+// paid half as often), and with a 168-register budget a CU holds three
+// workgroups. On MI355X the variance solve's updates ran at 124 TF/s staged
+// through registers (118 with 32-deep slabs and two workgroups); the direct
+// copies took a variance request at n = 24000 with 8192 columns from 155.4 to
+// 143.8 ms, with the FP64 residual product's, and the mixed request at
+// n = 32768 from 406.8 to 398.0.
 #include "kernels.hpp"
 
 namespace gpamd::k
@@ -20,10 +24,6 @@ namespace
 {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
-// staging registers of the global->LDS copy: a native vector type, so they
-// stay in registers (the HIP float4 struct ends up in scratch here)
-typedef float f4 __attribute__((ext_vector_type(4)));
-
 constexpr int THREADS = 256;
 
 // Tile shapes: B x B elements of C per workgroup, one quarter per wavefront,
@@ -34,8 +34,8 @@ struct Tile
 {
     static constexpr int BM = B, BK = D;
     static constexpr int Q = B / 2, NI = B / 32;        // a wavefront's quarter, in elements and 16-wide blocks
-    static constexpr int LPT = D * B / (THREADS * 4);  // 16-byte loads per thread per operand slab
-    static constexpr int KS = B + 16;  // floats per LDS k-row: the 4 k-slots of a read hit disjoint banks
+    static constexpr int LPT = D * B / (THREADS * 4);  // 16-byte copies per lane per operand slab
+    static constexpr int SLAB = D * B;                 // floats of LDS per slab
 };
 using Large = Tile<128, 16>;
 using Small = Tile<64, 32>;
@@ -63,22 +63,56 @@ struct Params32
     int tiles;     // capped: tiles holding part of the update
 };
 
-// Element offsets (within one slab) of this thread's LPT 16-byte loads,
-// clamped to the operand's last group of four; rows past the edge only feed
-// accumulators the epilogue never stores.
+// One operand's slabs, copied from memory straight into LDS (no staging
+// registers, no LDS writes ahead of the products' reads): every copy moves
+// 16 bytes per lane to 1 KiB of consecutive LDS, that is 256 / BM k-rows, so
+// the rows cannot be padded. The four k-slots of a read fall into disjoint
+// banks because row k holds column c at c ^ 16 (k mod 4), which the lanes
+// arrange by choosing what they fetch. Columns past the operand's edge are
+// clamped to its last group of four; they only feed accumulators the
+// epilogue never stores.
 template <class S>
-__device__ __forceinline__ void slab_offsets(long ld, int rows, int tid, unsigned (&off)[S::LPT], int (&lds)[S::LPT])
+struct DirectSlab32
 {
-#pragma unroll
-    for (int s = 0; s < S::LPT; s++)
+    static constexpr int ROWS = 256 / S::BM;  // k-rows per copy
+    const float *p[S::LPT];  // what the lane fetches in each of its wavefront's copies
+    long step;               // from one slab to the next
+    int first;               // the wavefront's first copy
+
+    __device__ __forceinline__ void init(const float *origin, long ld, int rows, int tid)
     {
-        const int idx = tid + THREADS * s;
-        const int kk = idx / (S::BM / 4);         // 0..BK-1
-        const int col = (idx % (S::BM / 4)) * 4;  // 0..BM-4
-        off[s] = static_cast<unsigned>(kk * ld + min(col, rows - 4));
-        lds[s] = kk * S::KS + col;
+        step = S::BK * ld;
+        first = __builtin_amdgcn_readfirstlane(tid >> 6) * S::LPT;
+        const int kk = (tid & 63) / (S::BM / 4), c = (tid & 63) % (S::BM / 4) * 4;
+#pragma unroll
+        for (int s = 0; s < S::LPT; s++)
+        {
+            const int k = (first + s) * ROWS + kk;
+            p[s] = origin + k * ld + min(c ^ 16 * (k & 3), rows - 4);
+        }
     }
-}
+
+    // T: 16-byte aligned LDS; p moves on to the next slab
+    __device__ __forceinline__ void fetch(float *T)
+    {
+#pragma unroll
+        for (int s = 0; s < S::LPT; s++)
+        {
+            using lds_ptr = __attribute__((address_space(3))) float *;
+            const unsigned dst = static_cast<unsigned>(reinterpret_cast<unsigned long>((lds_ptr)(T + (first + s) * 256)));
+            // no output register: the data goes to LDS at m0 + 16 lane; a
+            // write of m0 needs one wait state before its use
+            asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                         :
+                         : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(p[s])
+                         : "memory");
+            p[s] += step;
+        }
+    }
+
+    // this wavefront's copies are in LDS (a barrier shows them to the others)
+    static __device__ __forceinline__ void landed() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+};
 
 template <class S>
 __device__ __forceinline__ void mfma_slab32(const float *As, const float *Bs, int wr, int wc, int lm, int lk, v4f (&acc)[S::NI][S::NI])
@@ -89,10 +123,10 @@ __device__ __forceinline__ void mfma_slab32(const float *As, const float *Bs, in
         float a[S::NI], b[S::NI];
 #pragma unroll
         for (int i = 0; i < S::NI; i++)
-            a[i] = As[(kq * 4 + lk) * S::KS + wr * S::Q + i * 16 + lm];
+            a[i] = As[(kq * 4 + lk) * S::BM + ((wr * S::Q + i * 16) ^ 16 * lk) + lm];
 #pragma unroll
         for (int j = 0; j < S::NI; j++)
-            b[j] = Bs[(kq * 4 + lk) * S::KS + wc * S::Q + j * 16 + lm];
+            b[j] = Bs[(kq * 4 + lk) * S::BM + ((wc * S::Q + j * 16) ^ 16 * lk) + lm];
 #pragma unroll
         for (int i = 0; i < S::NI; i++)
 #pragma unroll
@@ -146,9 +180,9 @@ __device__ __forceinline__ void store_quarter32(const Params32<TC> &p, const v4f
 // part 0: the tile's whole K range; parts 1 and 2: its first and second
 // half (in slabs), for C -= updates only.
 template <class S, class TC>
-__device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long c0, float (*As)[S::BK * S::KS], float (*Bs)[S::BK * S::KS], int part = 0)
+__device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long c0, float (*As)[S::SLAB], float (*Bs)[S::SLAB], int part = 0)
 {
-    constexpr int BM = S::BM, BK = S::BK, LPT = S::LPT, NI = S::NI;
+    constexpr int BM = S::BM, BK = S::BK, NI = S::NI;
     const int rows_a = static_cast<int>(min(static_cast<long>(BM), p.M - r0));
     const int rows_b = static_cast<int>(min(static_cast<long>(BM), p.N - c0));
 
@@ -164,61 +198,35 @@ __device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long
         for (int j = 0; j < NI; j++)
             acc[i][j] = v4f{ 0.0f, 0.0f, 0.0f, 0.0f };
 
-    unsigned oa[LPT], ob[LPT];
-    int la[LPT], lb[LPT];
-    slab_offsets<S>(p.lda, rows_a, tid, oa, la);
-    slab_offsets<S>(p.ldb, rows_b, tid, ob, lb);
     const int kmax = p.k_to_row ? static_cast<int>(min(static_cast<long>(p.K), r0 + BM)) : p.K;
     const int kmin = p.k_from_row ? static_cast<int>(min(static_cast<long>(kmax), r0)) : 0;
     const int half = (kmax / BK / 2) * BK;
     const int k0 = part == 2 ? half : kmin, k1 = part == 1 ? half : kmax;
-    const float *ak = p.A + r0 + static_cast<long>(k0) * p.lda;
-    const float *bk = p.B + c0 + static_cast<long>(k0) * p.ldb;
-    const long astep = BK * p.lda, bstep = BK * p.ldb;
-
     if (k1 > k0)
     {
-    f4 ra[LPT], rb[LPT];
-#pragma unroll
-    for (int s = 0; s < LPT; s++)
-    {
-        ra[s] = *reinterpret_cast<const f4 *>(ak + oa[s]);
-        rb[s] = *reinterpret_cast<const f4 *>(bk + ob[s]);
-    }
-#pragma unroll
-    for (int s = 0; s < LPT; s++)
-    {
-        *reinterpret_cast<f4 *>(&As[0][la[s]]) = ra[s];
-        *reinterpret_cast<f4 *>(&Bs[0][lb[s]]) = rb[s];
-    }
-    __syncthreads();
-
-    int buf = 0;
-    const int steps = (k1 - k0) / BK;
-    for (int t = 1; t < steps; t++)
-    {
-        ak += astep;
-        bk += bstep;
-#pragma unroll
-        for (int s = 0; s < LPT; s++)
-        {
-            ra[s] = *reinterpret_cast<const f4 *>(ak + oa[s]);
-            rb[s] = *reinterpret_cast<const f4 *>(bk + ob[s]);
-        }
-        // the next slab's loads stay ahead of this slab's products
-        __builtin_amdgcn_sched_barrier(0);
-        mfma_slab32<S>(As[buf], Bs[buf], wr, wc, lm, lk, acc);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int s = 0; s < LPT; s++)
-        {
-            *reinterpret_cast<f4 *>(&As[buf ^ 1][la[s]]) = ra[s];
-            *reinterpret_cast<f4 *>(&Bs[buf ^ 1][lb[s]]) = rb[s];
-        }
+        DirectSlab32<S> da, db;
+        da.init(p.A + r0 + static_cast<long>(k0) * p.lda, p.lda, rows_a, tid);
+        db.init(p.B + c0 + static_cast<long>(k0) * p.ldb, p.ldb, rows_b, tid);
+        da.fetch(As[0]);
+        db.fetch(Bs[0]);
+        da.landed();
         __syncthreads();
-        buf ^= 1;
-    }
-    mfma_slab32<S>(As[buf], Bs[buf], wr, wc, lm, lk, acc);
+
+        int buf = 0;
+        const int steps = (k1 - k0) / BK;
+        for (int t = 1; t < steps; t++)
+        {
+            da.fetch(As[buf ^ 1]);
+            db.fetch(Bs[buf ^ 1]);
+            // the copies stay ahead of this slab's products
+            __builtin_amdgcn_sched_barrier(0);
+            mfma_slab32<S>(As[buf], Bs[buf], wr, wc, lm, lk, acc);
+            __builtin_amdgcn_sched_barrier(0);
+            da.landed();
+            __syncthreads();
+            buf ^= 1;
+        }
+        mfma_slab32<S>(As[buf], Bs[buf], wr, wc, lm, lk, acc);
     }
 
     // Accumulator layout of the 16x16x4 f32 MFMA on gfx950: lane holds
@@ -237,8 +245,8 @@ __device__ __forceinline__ void gemm_tile32(const Params32<TC> &p, long r0, long
 template <class S, int ROLE>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_gemm_f32_solve(Params32<float> p)
 {
-    __shared__ float As[2][S::BK * S::KS];
-    __shared__ float Bs[2][S::BK * S::KS];
+    __shared__ alignas(16) float As[2][S::SLAB];
+    __shared__ alignas(16) float Bs[2][S::SLAB];
     const unsigned gx = (p.N + S::BM - 1) / S::BM;
     gemm_tile32<S, float>(p, static_cast<long>(blockIdx.x / gx) * S::BM, static_cast<long>(blockIdx.x % gx) * S::BM, As, Bs);
 }
@@ -249,20 +257,11 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) vo
 template <class TC>
 __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) void k_gemm_f32_tn(Params32<TC> p)
 {
-    __shared__ float As[2][Large::BK * Large::KS];
-    __shared__ float Bs[2][Large::BK * Large::KS];
+    __shared__ alignas(16) float As[2][Large::SLAB];
+    __shared__ alignas(16) float Bs[2][Large::SLAB];
     const int gx = (p.N + BM - 1) / BM;
     const int gy = (p.M + BM - 1) / BM;
-    if (p.max_wgs <= 0)
-    {
-        // one workgroup per tile, row-major; tiles above the band do nothing
-        const long r0 = static_cast<long>(blockIdx.x / gx) * BM, c0 = static_cast<long>(blockIdx.x % gx) * BM;
-        if (p.lower && r0 + (BM - 1) + p.diag_off < c0)
-            return;
-        gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 0);
-        return;
-    }
-    // Capped: the tiles holding part of the update (for a lower update, those
+    // The tiles holding part of the update (for a lower update, those
     // touching the band) are numbered row by row, neighbours in flight
     // together. With a queue, each workgroup takes the next tile number from
     // a device counter when it is ready (one that starts late or shares its
@@ -270,7 +269,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) vo
     // updates the tiles numbered G/2 .. G-1 run as two K halves, the second
     // when the workgroup has nothing else left, so the two workgroups of a
     // CU do not reach their epilogues together; the choice depends only on
-    // tile numbers, so rounding does not depend on scheduling.
+    // tile numbers, so rounding does not depend on scheduling. An uncapped
+    // launch has a workgroup per tile and splits none.
     __shared__ int next;
     const int G = gridDim.x;
     long first_r = -1, first_c = 0;  // this workgroup's deferred second half
@@ -281,63 +281,54 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(3))) vo
         const long last = static_cast<long>(tr) * BM + (BM - 1) + p.diag_off;
         return last < 0 ? 0 : static_cast<int>(min(static_cast<long>(gx), last / BM + 1));
     };
-    auto run = [&](int t, long r0, long c0)
+    // one loop, one copy of the tile's code: with a copy for each way to take
+    // a tile the kernel spilled 103 registers (now 32, around the epilogue)
+    int tr = 0, row_first = 0, nc = gy > 0 ? row_tiles(0) : 0;  // the current tile row; tile numbers only grow
+    for (int t = blockIdx.x;; t += G)
     {
-        if (p.set || t < G / 2 || t >= G)
-            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 0);
-        else if (first_r < 0)
+        if (p.queue)
         {
-            first_r = r0;
-            first_c = c0;
-            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 1);
-        }
-        else
-        {
-            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 1);
-            __syncthreads();
-            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, 2);
-        }
-    };
-    if (p.queue)
-    {
-        int tr = 0, row_first = 0, nc = gy > 0 ? row_tiles(0) : 0;
-        for (;;)
-        {
-            __syncthreads();  // the previous tile's LDS reads and `next` reads are done
+            __syncthreads();  // the previous tile's `next` reads are done
             if (threadIdx.x == 0)
                 next = atomicAdd(p.queue, 1);
             __syncthreads();
-            const int t = next;
-            if (t >= p.tiles)
-                break;
+            t = __builtin_amdgcn_readfirstlane(next);
+        }
+        const bool done = t >= p.tiles;
+        if (done && first_r < 0)
+            break;
+        long r0 = first_r, c0 = first_c;
+        int part = 2, last = 2;  // with no other tile left: the deferred half
+        if (!done)
+        {
             while (t >= row_first + nc && tr + 1 < gy)
             {
                 row_first += nc;
                 nc = row_tiles(++tr);
             }
-            run(t, static_cast<long>(tr) * BM, static_cast<long>(t - row_first) * BM);
-        }
-    }
-    else
-    {
-        int rem = blockIdx.x;  // this workgroup's next tile, counted from the current row's first
-        int row_first = 0;
-        for (int tr = 0; tr < gy; tr++)
-        {
-            const int nc = row_tiles(tr);
-            for (; rem < nc; rem += G)
+            r0 = static_cast<long>(tr) * BM;
+            c0 = static_cast<long>(t - row_first) * BM;
+            const bool whole = p.set || p.max_wgs <= 0 || t < G / 2 || t >= G;
+            part = whole ? 0 : 1;
+            last = part;
+            if (!whole && first_r >= 0)
+                last = 2;  // a second split tile for this workgroup: both halves now
+            else if (!whole)
             {
-                __syncthreads();  // the previous tile's last slab has been read by every wavefront
-                run(row_first + rem, static_cast<long>(tr) * BM, static_cast<long>(rem) * BM);
+                first_r = r0;
+                first_c = c0;
             }
-            rem -= nc;
-            row_first += nc;
         }
-    }
-    if (first_r >= 0)
-    {
-        __syncthreads();
-        gemm_tile32<Large, TC>(p, first_r, first_c, As, Bs, 2);
+        // the same for all lanes: the tile's addresses stay in scalar registers
+        r0 = __builtin_amdgcn_readfirstlane(static_cast<int>(r0));
+        c0 = __builtin_amdgcn_readfirstlane(static_cast<int>(c0));
+        for (; part <= last; part++)
+        {
+            __syncthreads();  // the previous tile's last slab has been read by every wavefront
+            gemm_tile32<Large, TC>(p, r0, c0, As, Bs, part);
+        }
+        if (done)
+            break;
     }
 }
 
@@ -400,7 +391,7 @@ static void check_f32(const Params32<TC> &p)
     require(p.M % 4 == 0 && p.N % 4 == 0 && p.lda % 4 == 0 && p.ldb % 4 == 0
                 && reinterpret_cast<uintptr_t>(p.A) % 16 == 0 && reinterpret_cast<uintptr_t>(p.B) % 16 == 0,
             "FP32 product: operand rows must come in aligned groups of four");
-    require(static_cast<long>(Small::BK) * std::max(p.lda, p.ldb) + BM < (1L << 31), "FP32 product: operand too tall");
+    require(static_cast<long>(Large::BK) * std::max(p.lda, p.ldb) + BM < (1L << 31), "FP32 product: operand too tall");
 }
 
 void gemm_f32_trailing(hipStream_t s, const float *P, long ldp, long a_off, long b_off, double *C, long ldc, int M, int N, int K, long diag_off,
@@ -421,13 +412,14 @@ void gemm_f32_trailing(hipStream_t s, const float *P, long ldp, long a_off, long
     }
     if (active == 0)
         return;
-    p.tiles = static_cast<int>(std::min(active, (1L << 30)));
-    if (p.max_wgs >= active)
+    require(active < (1L << 30), "FP32 product: too many tiles");
+    p.tiles = static_cast<int>(active);
+    if (p.max_wgs <= 0 || p.max_wgs >= active)
     {
-        p.max_wgs = 0;  // the cap does not bind: one workgroup per tile
+        p.max_wgs = 0;  // no cap, or one that does not bind: one workgroup per tile
         p.queue = nullptr;
     }
-    dim3 grid(static_cast<unsigned>(p.max_wgs > 0 ? p.max_wgs : gx * gy));
+    dim3 grid(static_cast<unsigned>(p.max_wgs > 0 ? p.max_wgs : p.tiles));
     hipLaunchKernelGGL(k_gemm_f32_tn<double>, grid, dim3(THREADS), 0, s, p);
     GP_CHECK_LAUNCH();
 }
@@ -442,7 +434,8 @@ void gemm_f32_trailing(hipStream_t s, const float *P, long ldp, long a_off, long
 // 2000 / always): n = 12000, 300 columns 7.63 / 4.85 / 4.85 / 4.84 ms,
 // 1500 columns 11.55 / 10.03 / 9.85 / 9.84, 8192 columns 42.4 / 41.7 / 41.6 /
 // 41.7; n = 24000, 700 columns 22.95 / - / 18.58 / 18.24 / 18.26, 8192
-// columns 155.9 / - / 155.8 / 155.4 / 158.1. A diagonal step at 1536 columns
+// columns 155.9 / - / 155.8 / 155.4 / 158.1 (slabs still staged through
+// registers; since then 4.46, 9.11, 38.8, 16.99 and 143.8). A diagonal step at 1536 columns
 // went from 53 to 18 us, a third of that from leaving out the half of W_J
 // that is zero.
 constexpr long SMALL_TILE_LIMIT = 2048;
