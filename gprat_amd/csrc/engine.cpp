@@ -541,8 +541,6 @@ static void flow_solve(Context &c, const double *L, long lda, int n_pad, const d
     k::report(c.main, nullptr, 0, nullptr, c.info.get(), c.host_info);
 }
 
-void cholesky_fp64(Context &c, double *A, long lda, int n_pad, double *Winv) { cholesky(c, A, lda, n_pad, Winv, false); }
-
 int panel_width(int n_pad) { return outer_block(n_pad); }
 
 void cholesky(Context &c, double *A, long lda, int n_pad, double *Winv, bool mixed, double *Wpanel, int extra, double *X, int unit)

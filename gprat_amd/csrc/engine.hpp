@@ -271,7 +271,6 @@ struct Batch
 // Algorithms (engine.cpp)
 long padded(long n);
 long leading_dim(long n_pad);
-void cholesky_fp64(Context &c, double *A, long lda, int n_pad, double *Winv);
 // mixed: FP32 matrix-core trailing updates (FP64 panels and diagonal blocks).
 // Wpanel (optional): receives the k-major inverses of the panels' diagonal
 // blocks, panel_width(n_pad) wide, block k at Wpanel + k * width^2.
