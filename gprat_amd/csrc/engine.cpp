@@ -484,7 +484,7 @@ const Context::PanelPlanDev &Context::cached_plan(long key, const std::function<
 // the work per column, n (n / 3 + rows that ride along; identity rows
 // average a third), outgrows the difference. Measured on MI355X (panels /
 // dataflow, ms):
-//   fit       n = 1024 0.80 / 0.39, 4096 3.5 / 1.9, 8192 8.9 / 6.4, 10240 12.7 / 11.0, 12288 18.3 / 18.4
+//   fit       n = 1024 0.76 / 0.37, 4096 3.5 / 1.9, 8192 8.7 / 6.3, 10240 12.5 / 11.0, 12288 18.1 / 18.2
 //   one call  n = 6144 m = 1536 6.4 / 4.6, m = 6144 8.8 / 9.1; n = 8192 m = 2048 10.4 / 9.6, m = 8192 16.7 / 21.0;
 //             n = 10240 m = 640 13.2 / 12.4, m = 2560 16.2 / 17.7
 //   gradient  n = 4096 4.8 / 2.8, 8192 14.9 / 13.9, 10240 23.9 / 26.4

@@ -30,9 +30,10 @@
 //
 // Measured on MI355X: a step of the chain takes 14.5 us when nothing else runs
 // (factor 8, the two products 2.9, stores and hand-over 2.5), 25 to 40 us
-// beside a full device; n = 1024 / 2048 / 4992 / 8192 factored in 0.26 / 0.67 /
-// 2.2 / 5.8 ms (panel schedule: 0.70 / 1.5 / 4.1 / 8.6), the last at 32 TF/s:
-// a 64x64 tile's products read 64 KB of operands for 0.5 MFLOP.
+// beside a full device. A fit (assembly and alpha included) at n = 1024 / 2048 /
+// 4992 / 8192 takes 0.37 / 0.69 / 2.34 / 6.30 ms (panel schedule: 0.76 / 1.59 /
+// 4.35 / 8.72), the last's factorisation at 32 TF/s: a 64x64 tile's products
+// read 64 KB of operands for 0.5 MFLOP.
 #include <algorithm>
 #include <climits>
 
