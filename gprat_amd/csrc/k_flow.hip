@@ -25,8 +25,8 @@
 // counts too): a tile needs progress[i] > k and progress[j] > k for its k-th
 // product and progress[j] > j for W_jj. applied[r][c] counts the panels
 // subtracted from tile (r, c). Results are written with ordinary stores, made
-// visible by an agent-scope release before the counter moves, and read after
-// an agent-scope acquire.
+// visible by a write-back of the L2 that has ended before the counter moves
+// (publish), and read after an agent-scope acquire.
 //
 // Measured on MI355X: a step of the chain takes 14.5 us when nothing else runs
 // (factor 8, the two products 2.9, stores and hand-over 2.5), 25 to 40 us
@@ -118,14 +118,23 @@ __device__ __forceinline__ int wait_for(const FlowArgs &a, const int *p, const i
 }
 
 // This workgroup's stores are visible to whoever sees the counter at
-// `value`: every wavefront's have reached the L2 at the barrier, and the
-// release writes the L2 back.
+// `value`: every wavefront's have reached the L2 at the barrier, and the L2 is
+// written back before the counter moves. The write-back and the wait for it
+// are written out in one piece: the compiler's release store (clang of ROCm
+// 7.2) leaves that wait out wherever it knows of no other vector memory
+// operation in flight, as it did after the chain's L(j + 1, j). The counter
+// then overtook the tile: beside other kernels, whose dirty lines make a
+// write-back long, the next diagonal step read old elements of it (a fit of
+// n = 9000 was off by 3e-6 with requests of a server in flight).
 __device__ __forceinline__ void publish(int *p, int value)
 {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0)
-        __hip_atomic_store(p, value, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    {
+        asm volatile("buffer_wbl2 sc1\n\ts_waitcnt vmcnt(0)" ::: "memory");
+        __hip_atomic_store(p, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
 }
 
 // acc += A A^T beside mfma_nt_acc's A B^T, from the same staged rows.

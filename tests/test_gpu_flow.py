@@ -2,6 +2,7 @@
 the panel schedule at the sizes around its 64-wide tiles and its panels of
 eight (the tiled right-looking Cholesky of core/src/cpu/gp_algorithms.cpp)."""
 import os
+import threading
 from contextlib import contextmanager
 
 import numpy as np
@@ -147,3 +148,66 @@ def test_device_memory_in_and_out(ctx, n):
     assert all(np.array_equal(h, d.numpy()) for h, d in zip(a.predict(z, m), out))
     a.release()
     b.release()
+
+
+def first_difference(got, want):
+    """None, or the first quantity that is not bit-identical (a factor: its first 64x64 tile)."""
+    for name, w in want.items():
+        g = got[name]
+        if np.array_equal(g, w):
+            continue
+        at = np.argwhere(np.atleast_1d(g) != np.atleast_1d(w))
+        if name == "factor":
+            tiles = sorted({(int(c) // 64, int(r) // 64) for r, c in at})
+            return f"factor: {len(at)} entries, first in block column {tiles[0][0]}, block row {tiles[0][1]}"
+        return f"{name}: {len(at)} entries, first at {at[0].tolist()}"
+    return None
+
+
+def test_results_do_not_depend_on_other_launches():
+    """Two contexts in two threads: while their dataflow launches share the
+    device, each gives bit by bit what it gives alone."""
+    sizes, theta, m, rounds = (5003, 9000), (1.0, 1.0, 0.1), 33, 30
+    contexts = [capi.Context(0, 1) for _ in sizes]
+    problems = [datagen.gp_problem(n, m, 8) for n in sizes]
+
+    def results(k, factor):
+        n, c, (x, y, z) = sizes[k], contexts[k], problems[k]
+        out = {}
+        if factor:
+            out["factor"] = c.cholesky(x, theta, 1, n, 8)[0]
+        model = c.fit(x, y, n, 8, theta)
+        try:
+            out["loss"] = model.loss()
+            out["mean"], out["variance"] = model.predict(z, m)
+        finally:
+            model.release()
+        if n < 9000:
+            out["gradient"] = c.loss_gradient(x, y, theta, 1, n, 8)[1]
+        return out
+
+    differences = []
+
+    def work(k, alone, start):
+        try:
+            start.wait()
+            for i in range(rounds):
+                got = results(k, factor=i % 10 == 0)
+                d = first_difference(got, {q: alone[q] for q in got})
+                if d:
+                    differences.append(f"n = {sizes[k]}, pass {i}: {d}")
+        except Exception as e:
+            differences.append(f"n = {sizes[k]}: {e!r}")
+
+    try:
+        alone = [results(k, factor=True) for k in range(len(sizes))]
+        start = threading.Barrier(len(sizes))
+        threads = [threading.Thread(target=work, args=(k, alone[k], start)) for k in range(len(sizes))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+    finally:
+        for c in contexts:
+            c.close()
+    assert not differences, differences
