@@ -1229,7 +1229,7 @@ static void upload(Context &c, std::initializer_list<Upload> items)
 }
 
 // A result of `count` values on its way to the caller's memory: kernels write
-// to get(), send() goes before the call's last sync() and deliver() after it.
+// to get(), hand_out() passes it on.
 class Result
 {
   public:
@@ -1241,6 +1241,7 @@ class Result
             device_ = DevBuf<double>(c, count);
     }
     double *get() const { return staged_ ? staged_ : device_.get(); }
+    bool staged() const { return staged_ != nullptr; }
     void send()
     {
         if (!staged_)
@@ -1258,6 +1259,31 @@ class Result
     std::size_t count_;
     DevBuf<double> device_;
 };
+
+// Waits for the call's work and passes its results (null ones left out) to the
+// caller. pivots: they rest on a factorisation or solve whose outcome is not
+// known yet; if it failed, the caller's memory stays as it is.
+static void hand_out(Context &c, std::initializer_list<Result *> results, bool pivots)
+{
+    bool staged = true;
+    for (const Result *r : results)
+        staged = staged && (!r || r->staged());
+    if (pivots && !staged)
+    {
+        // a copy to the caller's own memory must not start before
+        c.sync();
+        check_pivots(c);
+    }
+    for (Result *r : results)
+        if (r)
+            r->send();
+    c.sync();
+    if (pivots)
+        check_pivots(c);
+    for (const Result *r : results)
+        if (r)
+            r->deliver();
+}
 
 static void check_training(const double *x, std::size_t x_len, int n, int r, const double *theta, int precision)
 {
@@ -1532,7 +1558,7 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
     }
     side.done();
     DevBuf<double> rows;
-    bool solved_here = false;  // by a dataflow launch: its completion is checked below
+    bool solved_here = false;  // by a dataflow launch, whose completion is checked
     if (var && m.mixed && m.refine_variance)
     {
         const int m_pad = static_cast<int>(round_up(mt, 64));
@@ -1580,15 +1606,7 @@ void predict_view(const FactorView &m, const double *z, std::size_t z_len, int m
         k::variance_finish(c.main, colsq.get(), m.sek.vertical, mt, vars->get());
     }
     side.join();
-    means.send();
-    if (vars)
-        vars->send();
-    c.sync();
-    means.deliver();
-    if (vars)
-        vars->deliver();
-    if (solved_here)
-        check_pivots(c);
+    hand_out(c, { &means, vars ? &*vars : nullptr }, solved_here);
 }
 
 // Mean and the whole latent posterior covariance Sigma = K** - V^T V,
@@ -1638,9 +1656,12 @@ void predict_full_cov_view(const FactorView &m, const double *z, std::size_t z_l
             Timed t(c, c.main, "trsm");
             k::subtract_row_products(c.main, V.get(), m.lda, m.n_pad, S.get(), m_pad, m_pad, part.get());
         }
-        download_square(c, S.get(), m_pad, mt, cov);
         if (how == ForwardSolve::OneLaunch)
+        {
+            c.sync();
             check_pivots(c);
+        }
+        download_square(c, S.get(), m_pad, mt, cov);
         return;
     }
     DevBuf<double> B(c, static_cast<std::size_t>(m.n_pad) * m_pad), S(c, static_cast<std::size_t>(m_pad) * m_pad);
@@ -1772,12 +1793,7 @@ void predict_with_uncertainty_once(Context &c, const double *x, std::size_t x_le
         Timed t(c, c.main, "mean");
         k::rows_mean_variance(c.main, rows, m.lda, mt, m.n_pad, yrow, m.sek.vertical, means.get(), vars.get());
     }
-    means.send();
-    vars.send();
-    c.sync();
-    check_pivots(c);
-    means.deliver();
-    vars.deliver();
+    hand_out(c, { &means, &vars }, true);
 }
 
 FactorView view(const Model &m)
@@ -2136,9 +2152,10 @@ void cholesky_tiles(Model &m, int T, int b, double *out)
     const std::size_t count = static_cast<std::size_t>(T) * (T + 1) / 2 * b * b;
     DevBuf<double> d(c, count);
     k::gather_tiles(c.main, m.L.get(), m.lda, m.x.get(), m.r, m.sek, T, b, d.get());
+    c.sync();
+    check_pivots(c);  // a factor that failed leaves the caller's array as it is
     GP_HIP(hipMemcpyAsync(out, d.get(), count * sizeof(double), hipMemcpyDefault, c.main));
     c.sync();
-    check_pivots(c);
 }
 
 }  // namespace gpamd

@@ -110,6 +110,30 @@ def test_first_failing_pivot(ctx, column):
     assert ctx.cholesky(u, (0.3, 1.0, 1e-3), 1, n, r).shape == (1, n, n)
 
 
+@pytest.mark.parametrize("n", [300, 1600])
+def test_a_failed_factorisation_leaves_the_outputs(ctx, n):
+    """Not positive definite: host arrays, arrays larger than the staging (65536
+    test points) and device buffers keep what they held."""
+    r, theta = 4, (0.3, 1.0, -1e-3)
+    u = np.arange(n + r - 1) * 10.0
+    u[n - 50:n - 50 + r] = u[:r]  # as above: the pivot of column n - 50 is about 2 * noise < 0
+    y, t = np.zeros(n), np.array(theta)
+    L, D = capi.lib(), capi._dptr
+    tiles = np.full(n * n, 7.5)
+    assert L.gprat_cholesky(ctx.handle, D(u), u.size, D(t), 1, n, r, D(tiles)) == capi.ERR_NOT_SPD
+    assert np.all(tiles == 7.5)
+    for m in (65, 65600):
+        z = np.linspace(0.0, 1.0, m + r - 1)
+        mean, var = np.full(m, 7.5), np.full(m, 7.5)
+        args = (ctx.handle, D(u), u.size, D(y), y.size, D(z), z.size, D(t), 1, n, 1, m, r)
+        assert L.gprat_predict_with_uncertainty(*args, D(mean), D(var)) == capi.ERR_NOT_SPD
+        assert np.all(mean == 7.5) and np.all(var == 7.5)
+    out = ctx.device_array(np.full(65, 7.5)), ctx.device_array(np.full(65, 7.5))
+    with pytest.raises(capi.GpratError):
+        ctx.predict(u, y, np.linspace(0.0, 1.0, 65 + r - 1), theta, 1, n, 1, 65, r, variance=True, out=out)
+    assert all(np.all(d.numpy() == 7.5) for d in out)
+
+
 @pytest.mark.parametrize("n", [100, 769, 2049, 2500])
 @pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 64, 65, 200, 1100])
 def test_forward_solves_agree(ctx, n, m):
