@@ -101,11 +101,16 @@ struct DirectSlab32
             using lds_ptr = __attribute__((address_space(3))) float *;
             const unsigned dst = static_cast<unsigned>(reinterpret_cast<unsigned long>((lds_ptr)(T + (first + s) * 256)));
             // no output register: the data goes to LDS at m0 + 16 lane; a
-            // write of m0 needs one wait state before its use
+            // write of m0 needs one wait state before its use. m0 is named as
+            // written, so that a value of the compiler's there is set again
+            // (it is nobody's to preserve, which is what clang warns of)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
                          :
                          : "s"(__builtin_amdgcn_readfirstlane(dst)), "v"(p[s])
-                         : "memory");
+                         : "memory", "m0");
+#pragma clang diagnostic pop
             p[s] += step;
         }
     }
