@@ -1497,14 +1497,26 @@ enum class ForwardSolve
     OneLaunch,
     Blocked
 };
-static ForwardSolve forward_solve(const FactorView &m, int mt)
+static ForwardSolve forward_solve(int n_pad, bool inverses, int mt)
 {
-    const long size = static_cast<long>(m.n_pad) * round_up(mt, 64);
+    const long size = static_cast<long>(n_pad) * round_up(mt, 64);
     if (const char *e = std::getenv("GPRAT_FORWARD_SOLVE"))
-        return std::atoi(e) == 0 && m.Wpanel ? ForwardSolve::FewRows : (std::atoi(e) <= 1 ? ForwardSolve::OneLaunch : ForwardSolve::Blocked);
-    if (m.Wpanel && size <= 4L << 20)
+        return std::atoi(e) == 0 && inverses ? ForwardSolve::FewRows : (std::atoi(e) <= 1 ? ForwardSolve::OneLaunch : ForwardSolve::Blocked);
+    if (inverses && size <= 4L << 20)
         return ForwardSolve::FewRows;
     return size <= 10L << 20 ? ForwardSolve::OneLaunch : ForwardSolve::Blocked;
+}
+static ForwardSolve forward_solve(const FactorView &m, int mt) { return forward_solve(m.n_pad, m.Wpanel != nullptr, mt); }
+
+std::size_t solved_rows_bytes(int n_pad, long lda, bool inverses, int mt)
+{
+    const ForwardSolve how = forward_solve(n_pad, inverses, mt);
+    if (how == ForwardSolve::Blocked)
+        return 0;
+    const std::size_t rows = round_up(mt, 64), buffer = rows * static_cast<std::size_t>(lda) * sizeof(double);
+    if (how == ForwardSolve::FewRows)
+        return 2 * buffer;
+    return buffer + static_cast<std::size_t>(k::flow_counters(n_pad / 64, static_cast<int>(rows / 64))) * sizeof(int);
 }
 
 // K* L^-T (the rows of V^T) for mt test points by one of the row methods:

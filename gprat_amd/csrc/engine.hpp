@@ -324,6 +324,10 @@ void predict(Model &m, const double *z, std::size_t z_len, int mt, double *mean,
 // points, with the rows of K* and the targets factored below K.
 void predict_with_uncertainty_once(Context &c, const double *x, std::size_t x_len, const double *y, std::size_t y_len, int n, int r,
                                    const double theta[3], const double *z, std::size_t z_len, int mt, double *mean, double *var);
+// Device memory of the rows that predict_view's variance holds for mt test
+// points where it solves by rows (0 where it takes the blocked solve), for an
+// FP64 factor with or without the panels' kept inverses.
+std::size_t solved_rows_bytes(int n_pad, long lda, bool inverses, int mt);
 void predict_view(const FactorView &m, const double *z, std::size_t z_len, int mt, double *mean, double *var);
 // Predictive mean through the fixed per-GPU scratch: no device allocation.
 void predict_mean_noalloc(Model &m, const double *z, std::size_t z_len, int mt, double *mean);

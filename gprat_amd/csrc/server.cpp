@@ -228,10 +228,17 @@ std::size_t Server::predict_need(const Entry &e, int m) const
     const std::size_t mp = round_up(m, 64);
     const std::size_t blocks = (np + 255) / 256;
     const std::size_t splits = static_cast<std::size_t>(k::mean_splits(e.n, m));
-    // K*^T, the staged V block and the panel copy (panel width wide), block
-    // inverses built for a factor without kept ones, the mean's partial sums
+    // what every way to solve holds: the mean's partial sums, vectors
     const std::size_t bo = e.batched_path ? 256 : static_cast<std::size_t>(panel_width(static_cast<int>(np)));
-    std::size_t bytes = 8 * (np * mp + bo * mp + 4 * mp + blocks * 65536 + bo * np + splits * m + m + e.r) + (std::size_t(1) << 20);
+    const std::size_t vectors = 8 * (4 * mp + splits * m + m + e.r) + (std::size_t(1) << 20);
+    // the blocked solve: K*^T, the staged V block and the panel copy (panel
+    // width wide), block inverses built for a factor without kept ones
+    const std::size_t blocked = 8 * (np * mp + bo * mp + blocks * 65536 + bo * np);
+    // the row methods: K*'s rows, beside them the solved ones or the
+    // dataflow launch's counters
+    const long ld = e.batched_path ? static_cast<long>(np) : leading_dim(static_cast<long>(np));
+    const std::size_t rows = solved_rows_bytes(static_cast<int>(np), ld, !e.batched_path, m);
+    std::size_t bytes = std::max(blocked, rows) + vectors;
     if (!e.small && cfg_.precision == GPRAT_PRECISION_MIXED)
     {
         // FP64-refined variance: FP32 K*^T / solution, FP64 K*^T, solution

@@ -221,6 +221,23 @@ def test_predict_keeps_its_own_least_recently_used_factor():
     assert np.array_equal(p1["mean"], p2["mean"]) and np.array_equal(p1["var"], p2["var"])
 
 
+@pytest.mark.parametrize("n, m", [(1024, 4096), (2048, 2048), (1024, 64), (2048, 4096)])
+def test_predict_reserves_the_rows_it_solves(n, m):
+    """A predict by the few-row kernels holds two buffers of m rows of n values
+    (K*'s rows and the solved ones), by the dataflow solve one: the budget has
+    to know them."""
+    from gprat_amd import capi
+    x, y, z = _data(70, n, 8, m)
+    with capi.Server(0, slots=1, precision=capi.PRECISION_FP64) as srv:
+        f = srv.submit_fit(x, y, n, 8, (1.0, 1.0, 0.1))
+        assert srv.wait(f)["status"] == 0
+        resident = srv.stats()["resident_bytes"]
+        assert srv.wait(srv.submit_predict(f, z, m))["status"] == 0
+        stats = srv.stats()
+    buffers = 2 if n * m <= 4 << 20 else 1
+    assert stats["peak_bytes"] >= resident + 8 * buffers * n * m, stats
+
+
 def test_failures_are_per_request():
     from gprat_amd import capi
     x, y, z = _data(90, 600, 8, 10)
