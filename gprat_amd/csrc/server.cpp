@@ -262,19 +262,23 @@ double Server::cost(const Request &r, const Entry &e) const
 }
 
 // Cost model of the small-fit routing (milliseconds, FP64, n <= 2048),
-// measured on MI355X (host-timed, n = 256 .. 2048):
-// * a single-GP fit uses the whole device but is bound by its launches'
-//   latency, about linear in n (0.27 ms at n = 256, 1.89 ms at 2048);
+// measured on MI355X (host-timed, n = 128 .. 2048):
+// * a single-GP fit is one dataflow launch, bound by its chain of block
+//   columns, about linear in n (0.15 ms at n = 128, 0.41 at 1024, 0.75 at 2048
+//   on one slot). Slots overlap less than they count: 48 fits of n = 512 took
+//   12.5 ms on one slot, 6.9 on two, 5.2 on three, 4.3 on four, 4.0 on six
+//   (n = 2048: 35.9, 21.1, 15.9, 14.0, 15.8);
 // * a batched fit runs its GPs above n_pad 128 as level-synchronous launches
 //   (two per 64-row block of the largest GP), so it lasts as long as that
-//   chain of launches (0.34 ms for one GP of n = 256, 1.55 ms at 1024,
-//   4.67 ms at 2048) plus the GPs' work at the batch's throughput (16 GPs of
-//   n = 2048: 5.51 ms).
-static double single_fit_ms(int n) { return 0.05 + 0.00092 * n; }
+//   chain of launches (0.29 ms for one GP of n = 256, 1.10 ms at 1024,
+//   2.99 ms at 2048) plus the GPs' work at the batch's throughput (16 GPs of
+//   n = 2048: 3.6 ms, 64: 6.7 ms).
+static double single_fit_ms(int n) { return 0.11 + 0.00031 * n; }
+static double slot_overlap(int slots) { return std::min(2.6, 0.35 + 0.65 * slots); }
 static double batch_chain_ms(int n_max)
 {
     const double n = n_max;
-    return 0.14 + 5.37e-4 * n + 8.0e-7 * n * n;
+    return 0.115 + 5.5e-4 * n + 4.2e-7 * n * n;
 }
 static double batch_work_ms(int n)
 {
@@ -286,7 +290,7 @@ static double batch_work_ms(int n)
 // from the small fits waiting at and after `first` (up to batch_max), or 0
 // for none. For each cut n_c, the fits with n <= n_c would take one batched
 // fit (batch_chain_ms(n_c) plus their work) against their single-GP times
-// spread over the slots; the cut with the largest saving wins (at least two
+// as the slots overlap them; the cut with the largest saving wins (at least two
 // fits). A lone small fit, or a few small fits that the slots finish
 // sooner one by one, take the single-GP path.
 int Server::batch_cut(std::deque<Request>::iterator first)
@@ -310,7 +314,7 @@ int Server::batch_cut(std::deque<Request>::iterator first)
         const int count = static_cast<int>(k) + 1;
         if (count < 2 || (k + 1 < ns.size() && ns[k + 1] == ns[k]))
             continue;
-        const double saving = single / std::min(count, cfg_.slots) - (batch_chain_ms(ns[k]) + work);
+        const double saving = single / slot_overlap(std::min(count, cfg_.slots)) - (batch_chain_ms(ns[k]) + work);
         if (saving > best)
         {
             best = saving;
