@@ -198,7 +198,10 @@ __device__ __forceinline__ void stage_difference(double *buf, const double (&s)[
 
 // The thread's index, hidden from the compiler: what follows from it is not
 // carried from task to task (the addresses of a task's block operations, kept
-// across the task loop, overflowed the registers).
+// across the task loop, filled 188 more registers). The factorisation still
+// spills 105 of its 256 registers: the diagonal task keeps addresses and
+// accumulators in scratch (440 bytes a lane). The launch on a given factor
+// spills none.
 __device__ __forceinline__ int own_thread()
 {
     int t = threadIdx.x;
